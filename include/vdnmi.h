@@ -98,6 +98,26 @@ int vdn_mxfp8_gemm_act_quantize(const void* a, const void* a_scales, int64_t mp,
                                 int act, void* q, void* scales, int64_t out_rows, int64_t n,
                                 uint32_t* nonfinite, void* stream);
 
+/*
+ * vdn_mxfp8_gemm and vdn_mxfp8_gemm_act_quantize with a caller's workspace (16-byte aligned,
+ * private to the call until it has run on `stream`; contents immaterial). With at least the
+ * bytes vdn_mxfp8_gemm_workspace reports, a problem with few tiles shares a tile's K steps
+ * between workgroups, whose fp32 partials the workspace holds; with fewer (or null) it runs as
+ * without. kind: 0 bf16 output, 1 with a residual, 2 producer (act 0 or 1), 3 SwiGLU (act 2);
+ * 0 bytes: the problem has no use for a workspace.
+ */
+int vdn_mxfp8_gemm_ws(const void* a, const void* a_scales, int64_t mp, const void* w,
+                      const void* w_scales, int64_t np, int64_t kp, const void* bias,
+                      const void* addend, int64_t ld_add, const void* residual, int64_t ld_res,
+                      const void* gate, void* out, int64_t out_rows, int64_t n, int64_t ldc,
+                      uint32_t* nonfinite, void* workspace, int64_t workspace_bytes, void* stream);
+int vdn_mxfp8_gemm_act_quantize_ws(const void* a, const void* a_scales, int64_t mp, const void* w,
+                                   const void* w_scales, int64_t np, int64_t kp, const void* bias,
+                                   int act, void* q, void* scales, int64_t out_rows, int64_t n,
+                                   uint32_t* nonfinite, void* workspace, int64_t workspace_bytes,
+                                   void* stream);
+int vdn_mxfp8_gemm_workspace(int64_t mp, int64_t np, int64_t kp, int kind, int64_t* bytes);
+
 /* ---------------------------------------------------------------------------------------
  * VDA linear-attention branch (D = 128). A 4-D operand "(f, h, s, c)" is addressed as
  * base + f*sf + h*sh + s*ss + c (element strides, channels contiguous); raw token-major

@@ -1,0 +1,120 @@
+"""The block-scaled GEMM's stream kernel (small and middle sizes) against the oracle.
+
+Shapes reach its 128- and 256-column tiles, whole tiles only, K steps shared between workgroups
+(alone and beside whole tiles), the rows left below whole waves of the large kernel, padded
+columns past the last 256-column tile, single and odd K steps and the last partial rows. Each is
+checked on sampled rows against the exactly dequantized float64 GEMM, within the accumulation
+bound of tests/test_mxfp8_gpu.py::test_gemm_gated_residual_epilogue, for the bf16, gated-residual
+and producer epilogues; without a workspace the same problem runs unshared.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import mxfp8 as om
+from vdn_amd import _lib
+from vdn_amd import mxfp8 as vm
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    (1, 128, 128),        # one tile, one K step
+    (77, 5120, 1152),     # few tiles: K shared, 9 steps in uneven parts
+    (130, 200, 384),      # an odd number of steps, n below its padding
+    (300, 1920, 640),     # padded N 1920: the last 256-column tile half past it
+    (512, 5120, 1024),    # 128-column tiles
+    (960, 5120, 768),     # 256-column tiles, one each
+    (1560, 5120, 1536),   # whole tiles and shared ones beside them
+    (2304, 7168, 384),    # more than one whole tile each
+    (3330, 5376, 1024),   # the large kernel, then the rows below its whole waves
+]
+
+
+def operands(m, n, k):
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16)
+    bias = (torch.randn(n, generator=g) * 0.5).to(torch.bfloat16)
+    gate = torch.randn(n, generator=g).to(torch.bfloat16)
+    res = torch.randn(m, n, generator=g).to(torch.bfloat16)
+    rows = np.unique(np.concatenate([np.arange(0, m, 128), np.arange(127, m, 128),
+                                     np.arange(max(0, m - 3), m)]))
+    wc, wn, _ = om.quantize(w.float().numpy())
+    ac, an, _ = om.quantize(x[torch.from_numpy(rows)].float().numpy())
+    y0 = om.bf16_round(om.gemm(ac, an, wc, wn, len(rows), n))
+    mag = om.gemm_magnitude(ac, an, wc, wn, len(rows), n)
+    y = om.bf16_round(y0 + bias.float().numpy()[None])
+    limit = om.bf16_ulp(y0) + om.bf16_ulp(y) + om.MFMA_ACCUMULATION_BOUND * mag
+    return x, w, bias, gate, res, rows, y, limit
+
+
+def check(got, rows, ref, limit):
+    got = got[torch.from_numpy(rows).to(got.device)].float().cpu().numpy().astype(np.float64)
+    err = np.abs(got - ref)
+    assert (err <= limit).all(), float((err / limit).max())
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_stream_gemm_matches_oracle(device, m, n, k):
+    x, w, bias, gate, res, rows, y, limit = operands(m, n, k)
+    q, s = vm.quantize_activation(x.to(device))
+    wq, ws = vm.quantize_activation(w.to(device))
+    b, g = bias.to(device), gate.to(device)
+    flag = torch.zeros(1, dtype=torch.int32, device=device)
+    store = torch.full((m + 5, n), 7.0, dtype=torch.bfloat16, device=device)
+    plain = vm.mxfp8_gemm(q, s, wq, ws, n, rows=m, bias=b, out=store[:m], nonfinite=flag)
+    assert bool((store[m:] == 7.0).all()), "rows past M are not written"
+    check(plain, rows, y, limit)
+    # gated residual, over the residual itself
+    out = res.to(device)
+    vm.mxfp8_gemm(q, s, wq, ws, n, rows=m, bias=b, out=out, residual=out, gate=g, nonfinite=flag)
+    gy = om.bf16_round(gate.float().numpy()[None] * y)
+    ref = om.bf16_round(res.float().numpy()[rows] + gy)
+    check(out, rows, ref, np.abs(gate.float().numpy())[None] * limit + om.bf16_ulp(gy) + om.bf16_ulp(ref))
+    assert int(flag.item()) == 0
+    # the producer form sums in the same order: the bytes of the separate passes
+    for act, fn in ((None, vm.launch_quantize), ("gelu_tanh", vm.launch_gelu_quantize)):
+        fq, fs = vm.mxfp8_gemm_act_quantize(q, s, wq, ws, n, rows=m, bias=b, act=act)
+        rq, rs = fn(plain)[:2]
+        assert torch.equal(fq, rq) and torch.equal(fs, rs), act
+    # the same problem without a workspace
+    again = torch.empty(m, n, dtype=torch.bfloat16, device=device)
+    if n % 8 == 0:
+        _lib.call("vdn_mxfp8_gemm", q.data_ptr(), s.data_ptr(), q.shape[0], wq.data_ptr(),
+                  ws.data_ptr(), wq.shape[0], q.shape[1], b.data_ptr(), None, 0, None, 0, None,
+                  again.data_ptr(), m, n, n, None, _lib.stream(again.device))
+        check(again, rows, y, limit)
+
+
+@pytest.mark.parametrize("m,f,k", [(77, 1280, 1152), (1560, 2560, 1536), (3330, 2816, 1024),
+                                   (260, 200, 128)])
+def test_stream_swiglu_matches_separate_passes(device, m, f, k):
+    """The SwiGLU producer against the same interleaved GEMM, regrouped, and the stand-alone
+    producer: the same bytes, also where K is shared."""
+    g = torch.Generator().manual_seed(m + f)
+    x = (torch.randn(m, k, generator=g) * 2).to(torch.bfloat16).to(device)
+    w, b = vm.interleave_swiglu((torch.randn(2 * f, k, generator=g) * 0.05).to(torch.bfloat16),
+                                torch.randn(2 * f, generator=g).to(torch.bfloat16))
+    q, s = vm.quantize_activation(x)
+    wq, ws = vm.quantize_activation(w.to(device))
+    fq, fs = vm.mxfp8_gemm_act_quantize(q, s, wq, ws, f, rows=m, bias=b.to(device), act="swiglu")
+    fp = wq.shape[0] // 2
+    y = vm.mxfp8_gemm(q, s, wq, ws, 2 * fp, rows=m, bias=b.to(device))
+    y = y.view(m, fp // 128, 2, 128).transpose(1, 2).reshape(m, 2, fp)[:, :, :f].reshape(m, 2 * f)
+    rq, rs, _ = vm.launch_swiglu_quantize(y)
+    assert torch.equal(fq, rq) and torch.equal(fs, rs)
+
+
+def test_stream_gemm_flags_nonfinite(device):
+    """An inf in one row reaches the flag through whole and through shared tiles."""
+    for m, n, k in ((77, 1280, 1152), (512, 5120, 256)):
+        x = torch.ones(m, k, dtype=torch.bfloat16)
+        x[m - 1] = 3e38
+        q, s = vm.quantize_activation(x.to(device))
+        wq, ws = vm.quantize_activation(torch.ones(n, k, dtype=torch.bfloat16, device=device))
+        flag = torch.zeros(1, dtype=torch.int32, device=device)
+        vm.mxfp8_gemm(q, s, wq, ws, n, rows=m, nonfinite=flag)
+        assert int(flag.item()) != 0
+        flag.zero_()
+        vm.mxfp8_gemm(q, s, wq, ws, n, rows=m - 1, nonfinite=flag)   # that row is no output now
+        assert int(flag.item()) == 0

@@ -21,14 +21,12 @@
 //   * workgroup ids are remapped so consecutive tiles land on the same XCD (dispatch is
 //     round-robin over the 8 XCDs) and tiles are walked in GROUP_M-row groups, which keeps
 //     each XCD's L2 working set to a few A row-panels and W column-panels.
-#include "mxfp8_common.h"
+#include "mxfp8_gemm.h"
 
 #include <type_traits>
 
 namespace vdn {
 namespace {
-
-constexpr int kBK = 128;
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef const __attribute__((address_space(1))) void global_void_t;
@@ -39,65 +37,6 @@ __device__ __forceinline__ void load_to_lds16(const void* src, void* lds_wave_ba
 
 __device__ __forceinline__ void load_to_lds4(const void* src, void* lds_wave_base) {
   __builtin_amdgcn_global_load_lds((global_void_t*)src, (lds_void_t*)lds_wave_base, 4, 0, 0);
-}
-
-// SWIZZLE_32_4_4 keeps the scale dwords (4 K-blocks of one 128-K step) of a 128-row block
-// in one contiguous 512-byte run: row r's dword sits at 16 (r % 32) + 4 ((r % 128) / 32)
-// of it. The run of block b for K step ks starts at (b * col_tiles + ks) * 512.
-__device__ __forceinline__ int scale_in_block(int r) { return (r & 31) * 16 + ((r & 127) >> 5) * 4; }
-
-// Epilogue of one output element y (the bf16-rounded accumulator), in this order:
-//   y = bf16(y + bias[c])                    (bias: nullable, [n])
-//   y = bf16(addend[r, c] + y)               (addend: nullable)
-//   y = bf16(residual[r, c] + bf16(gate[c] * y))   (residual: nullable; gate nullable = 1)
-// `out` may alias `addend` or `residual`: every element is read and written by one lane.
-struct Epilogue {
-  const uint16_t* bias;
-  const uint16_t* addend;
-  int64_t ld_add;
-  const uint16_t* residual;
-  int64_t ld_res;
-  const uint16_t* gate;
-  uint16_t* out;
-  int64_t ldc;
-  uint32_t* nonfinite;
-  int vec;  // 16-byte accesses: n, every leading dimension and pointer 8-element aligned
-  // Producer mode (q_out non-null): instead of bf16 `out`, y = bf16(bf16(acc) + bias) goes
-  // through `act` (0 none, 1 GELU-tanh, rounded to bf16) and is stored as MXFP8 codes
-  // q_out [mp, kp_out] + swizzled scales s_out, exactly what the producer kernels write
-  // for that bf16 matrix. Rows >= out_rows and columns >= n are stored as zero.
-  uint8_t* q_out;
-  uint8_t* s_out;
-  int64_t kp_out;
-  int act;
-};
-
-// Epilogue arithmetic of one element (see Epilogue).
-__device__ __forceinline__ float epilogue_value(float y, float b, float addend, float res, float gt,
-                                                const Epilogue& ep) {
-  if (ep.bias != nullptr) y = round_bf16(y + b);
-  if (ep.addend != nullptr) y = round_bf16(addend + y);
-  if (ep.residual != nullptr) {
-    const float t = ep.gate != nullptr ? round_bf16(gt * y) : y;
-    y = round_bf16(res + t);
-  }
-  return y;
-}
-
-__device__ __forceinline__ void unpack4(const u32x2 w, float* f) {
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    f[2 * i] = __uint_as_float(w[i] << 16);
-    f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-  }
-}
-
-__device__ __forceinline__ void unpack8(const u32x4 w, float* f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = bf16_bits_to_f32(static_cast<uint16_t>(w[i] & 0xffff));
-    f[2 * i + 1] = bf16_bits_to_f32(static_cast<uint16_t>(w[i] >> 16));
-  }
 }
 
 template <int BM, int BN, int WGM, int WGN>
@@ -337,34 +276,7 @@ mxfp8_gemm_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ As,
   constexpr int kPasses = BM / kRowsPerPass;
   constexpr int kBatch = kPasses < 8 ? kPasses : 8;
   static_assert(kPasses % kBatch == 0, "epilogue batching");
-  if (ep.q_out != nullptr) {
-    // Eight consecutive columns per lane; the four lanes of a 32-column block and the
-    // sixteen of a 128-column chunk are consecutive lanes of one row (kChunksPerRow is a
-    // multiple of 16), which is the lane layout quantize_store8 expects.
-    static_assert(kChunksPerRow % 16 == 0, "producer epilogue lane layout");
-    const int64_t chunk128 = (n0 >> 7) + (chunk >> 4);
-    // a 256-wide tile can reach past the padded output (rows >= mp, chunks >= kp_out / 128);
-    // both tests are uniform over the 16 lanes of a chunk
-    const bool chunk_in = chunk128 < (ep.kp_out >> 7);
-    for (int pass = 0; pass < kPasses; ++pass) {
-      const int r = pass * kRowsPerPass + tid / kChunksPerRow;
-      const int64_t row = m0 + r;
-      if (row >= mp || !chunk_in) continue;
-      float y[8];
-      unpack8(*reinterpret_cast<const u32x4*>(lds_raw + r * kStageStride + chunk * 16), y);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float v = 0.f;
-        if (row < out_rows && col + e < n) {
-          v = ep.bias != nullptr ? round_bf16(y[e] + bias8[e]) : y[e];
-          if (ep.act == 1) v = round_bf16(gelu_tanh(v));
-          bad = bad || !(fabsf(v) < INFINITY);
-        }
-        y[e] = v;
-      }
-      quantize_store8(y, tid & 15, row, chunk128, ep.kp_out, ep.q_out, ep.s_out);
-    }
-  } else if (ep.vec && col + 8 <= n) {
+  if (ep.vec && col + 8 <= n) {
     // Batches of kBatch rows: every load of a batch is issued before any arithmetic, so
     // the addend/residual latency is paid once per batch rather than once per row.
     for (int b0 = 0; b0 < kPasses; b0 += kBatch) {
@@ -424,7 +336,7 @@ mxfp8_gemm_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ As,
 }
 
 // ---------------------------------------------------------------------------------------
-// Persistent 256 x 256 kernel (the large-problem path).
+// Persistent 256 x 256 kernel (the large-problem path; plan_gemm in mxfp8_gemm_stream.hip chooses).
 //
 // One workgroup per CU walks its tiles (XCD-contiguous order as above) with one K-step
 // pipeline that runs across tile boundaries: step s of the workgroup's (tile, K step)
@@ -1043,6 +955,8 @@ constexpr int kPGroupM = 4;
 #define VDN_GEMM_HEAD 2
 #endif
 
+}  // namespace
+
 int cu_count() {
   static int cached[64];
   int dev = 0;
@@ -1055,48 +969,122 @@ int cu_count() {
   return cu;
 }
 
-int launch_persistent(const uint8_t* a, const uint8_t* as, int64_t mp, const uint8_t* w,
-                      const uint8_t* ws, int64_t np, int64_t kp, const Epilogue& ep,
-                      int64_t out_rows, int64_t n, hipStream_t stream) {
-  const int64_t tiles_m = (mp + kPTile - 1) / kPTile, tiles_n = (np + kPTile - 1) / kPTile;
-  if (tiles_m * tiles_n > (1ll << 31) - 1 || static_cast<int64_t>(kPTile) * kp >= (1ll << 31) ||
-      mp * kp / 32 >= (1ll << 31) || np * kp / 32 >= (1ll << 31))
-    return set_error(kUnsupported, "vdn_mxfp8_gemm: problem too large for 32-bit tile offsets");
+int launch_persistent(const GemmArgs& g, hipStream_t stream) {
+  const int64_t tiles_m = (g.mp + kPTile - 1) / kPTile, tiles_n = (g.np + kPTile - 1) / kPTile;
   const int64_t tiles = tiles_m * tiles_n;
   const int grid = static_cast<int>(tiles < cu_count() ? tiles : cu_count());
   const int tm = static_cast<int>(tiles_m), tn = static_cast<int>(tiles_n);
-  if (ep.q_out != nullptr && ep.act == 2)
-    hipLaunchKernelGGL((mxfp8_gemm_persistent_kernel<VDN_GEMM_HEAD, 3>), dim3(grid), dim3(256),
-                       0, stream, a, as, w, ws, mp, np, kp, ep, out_rows, n, tm, tn, kPGroupM);
-  else if (ep.q_out != nullptr)
-    hipLaunchKernelGGL((mxfp8_gemm_persistent_kernel<VDN_GEMM_HEAD, 2>), dim3(grid), dim3(256),
-                       0, stream, a, as, w, ws, mp, np, kp, ep, out_rows, n, tm, tn, kPGroupM);
-  else if (ep.residual != nullptr)
-    hipLaunchKernelGGL((mxfp8_gemm_persistent_kernel<VDN_GEMM_HEAD, 1>), dim3(grid), dim3(256),
-                       0, stream, a, as, w, ws, mp, np, kp, ep, out_rows, n, tm, tn, kPGroupM);
-  else
-    hipLaunchKernelGGL((mxfp8_gemm_persistent_kernel<VDN_GEMM_HEAD, 0>), dim3(grid), dim3(256),
-                       0, stream, a, as, w, ws, mp, np, kp, ep, out_rows, n, tm, tn, kPGroupM);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, g.a, g.as, g.w, g.ws, g.mp, g.np, g.kp, g.ep,
+                       g.out_rows, g.n, tm, tn, kPGroupM);
+  };
+  switch (gemm_mode(g.ep)) {
+    case 0: launch(mxfp8_gemm_persistent_kernel<VDN_GEMM_HEAD, 0>); break;
+    case 1: launch(mxfp8_gemm_persistent_kernel<VDN_GEMM_HEAD, 1>); break;
+    case 2: launch(mxfp8_gemm_persistent_kernel<VDN_GEMM_HEAD, 2>); break;
+    default: launch(mxfp8_gemm_persistent_kernel<VDN_GEMM_HEAD, 3>); break;
+  }
   return check_launch("vdn_mxfp8_gemm");
 }
 
+namespace {
+
+// 32-bit tile, scale and tile-count arithmetic of the GEMM kernels with tiles of up to
+// `tile_rows` rows.
+bool gemm_too_large(int64_t mp, int64_t np, int64_t kp, int64_t tile_rows) {
+  return (mp / 128) * (np / 128) > (1ll << 31) - 1 || tile_rows * kp >= (1ll << 31) ||
+         mp * kp / 32 >= (1ll << 31) || np * kp / 32 >= (1ll << 31);
+}
+
 template <int BM, int BN, int WGM, int WGN>
-int launch_gemm(const uint8_t* a, const uint8_t* as, int64_t mp, const uint8_t* w,
-                const uint8_t* ws, int64_t np, int64_t kp, const Epilogue& ep, int64_t out_rows,
-                int64_t n, hipStream_t stream) {
-  const int64_t tiles_m = (mp + BM - 1) / BM, tiles_n = (np + BN - 1) / BN;
-  if (tiles_m * tiles_n > (1ll << 31) - 1 || static_cast<int64_t>(BM) * kp >= (1ll << 31) ||
-      mp * kp / 32 >= (1ll << 31) || np * kp / 32 >= (1ll << 31))
-    return set_error(kUnsupported, "vdn_mxfp8_gemm: problem too large for 32-bit tile offsets");
+int launch_gemm(const GemmArgs& g, hipStream_t stream) {
+  const int64_t tiles_m = (g.mp + BM - 1) / BM, tiles_n = (g.np + BN - 1) / BN;
   const int group_m = 8;
   hipLaunchKernelGGL((mxfp8_gemm_kernel<BM, BN, WGM, WGN>), dim3(tiles_m * tiles_n),
-                     dim3(WGM * WGN * 64), 0, stream, a, as, w, ws, mp, np, kp, ep, out_rows, n,
-                     static_cast<int>(tiles_m),
-                     static_cast<int>(tiles_n), group_m);
+                     dim3(WGM * WGN * 64), 0, stream, g.a, g.as, g.w, g.ws, g.mp, g.np, g.kp, g.ep,
+                     g.out_rows, g.n, static_cast<int>(tiles_m), static_cast<int>(tiles_n), group_m);
   return check_launch("vdn_mxfp8_gemm");
 }
 
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
+
+int gemm(const char* name, const void* a, const void* a_scales, int64_t mp, const void* w,
+         const void* w_scales, int64_t np, int64_t kp, const void* bias, const void* addend, int64_t ld_add,
+         const void* residual, int64_t ld_res, const void* gate, void* out, int64_t out_rows, int64_t n,
+         int64_t ldc, uint32_t* nonfinite, float* workspace, int64_t workspace_bytes, void* stream) {
+  if (a == nullptr || a_scales == nullptr || w == nullptr || w_scales == nullptr || out == nullptr)
+    return set_error(kInvalidArgument, "%s: null pointer argument", name);
+  if (mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128)
+    return set_error(kInvalidArgument, "%s: padded M/N/K must be positive multiples of 128", name);
+  if (n <= 0 || n > np || out_rows < 0 || out_rows > mp || ldc < n ||
+      (addend != nullptr && ld_add < n) || (residual != nullptr && ld_res < n))
+    return set_error(kInvalidArgument, "%s: invalid output geometry", name);
+  if (gate != nullptr && residual == nullptr)
+    return set_error(kInvalidArgument, "%s: a gate needs a residual", name);
+  if (!aligned(a, 16) || !aligned(w, 16) || !aligned(a_scales, 4) || !aligned(w_scales, 4))
+    return set_error(kInvalidArgument, "%s: code buffers need 16-byte, scales 4-byte alignment",
+                     name);
+  if (workspace != nullptr && (!aligned(workspace, 16) || workspace_bytes < 0))
+    return set_error(kInvalidArgument, "%s: the workspace needs 16-byte alignment", name);
+  if (out_rows == 0) return kOk;
+  const bool vec = n % 8 == 0 && ldc % 8 == 0 && aligned(out, 16) &&
+                   (bias == nullptr || aligned(bias, 16)) && (gate == nullptr || aligned(gate, 16)) &&
+                   (addend == nullptr || (ld_add % 8 == 0 && aligned(addend, 16))) &&
+                   (residual == nullptr || (ld_res % 8 == 0 && aligned(residual, 16)));
+  const bool large = mp >= 1024 && np >= 1024;
+  if (gemm_too_large(mp, np, kp, large ? 256 : 128))
+    return set_error(kUnsupported, "%s: problem too large for 32-bit tile offsets", name);
+  const GemmArgs g{static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(a_scales),
+                   static_cast<const uint8_t*>(w), static_cast<const uint8_t*>(w_scales), mp, np, kp,
+                   Epilogue{static_cast<const uint16_t*>(bias), static_cast<const uint16_t*>(addend),
+                            ld_add, static_cast<const uint16_t*>(residual), ld_res,
+                            static_cast<const uint16_t*>(gate), static_cast<uint16_t*>(out), ldc,
+                            nonfinite, vec ? 1 : 0, nullptr, nullptr, 0, 0},
+                   out_rows, n};
+  auto st = static_cast<hipStream_t>(stream);
+  // an addend, or rows that 16-byte accesses do not cover, take the general kernel
+  if (vec && addend == nullptr)
+    return launch_gemm_planned(g, gemm_mode(g.ep), workspace, workspace_bytes, st);
+  if (large) return launch_gemm<256, 256, 2, 2>(g, st);
+  return launch_gemm<128, 128, 2, 2>(g, st);
+}
+
+int gemm_act_quantize(const char* name, const void* a, const void* a_scales, int64_t mp, const void* w,
+                      const void* w_scales, int64_t np, int64_t kp, const void* bias, int act, void* q,
+                      void* scales, int64_t out_rows, int64_t n, uint32_t* nonfinite, float* workspace,
+                      int64_t workspace_bytes, void* stream) {
+  if (a == nullptr || a_scales == nullptr || w == nullptr || w_scales == nullptr || q == nullptr ||
+      scales == nullptr)
+    return set_error(kInvalidArgument, "%s: null pointer argument", name);
+  if (mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128)
+    return set_error(kInvalidArgument, "%s: padded M/N/K must be positive multiples of 128", name);
+  if (n <= 0 || n > np || out_rows < 0 || out_rows > mp)
+    return set_error(kInvalidArgument, "%s: invalid output geometry", name);
+  if (act != 0 && act != 1 && act != 2)
+    return set_error(kInvalidArgument, "%s: unknown activation %d", name, act);
+  if (!aligned(a, 16) || !aligned(w, 16) || !aligned(a_scales, 4) || !aligned(w_scales, 4) ||
+      !aligned(q, 16) || !aligned(scales, 4) || (bias != nullptr && !aligned(bias, 16)))
+    return set_error(kInvalidArgument, "%s: misaligned buffer", name);
+  if (workspace != nullptr && (!aligned(workspace, 16) || workspace_bytes < 0))
+    return set_error(kInvalidArgument, "%s: the workspace needs 16-byte alignment", name);
+  if (out_rows == 0) return kOk;
+  const int64_t kp_out = (n + 127) / 128 * 128;
+  // Every column chunk up to kp_out must be produced: the padded GEMM width covers it.
+  if (kp_out > np) return set_error(kInvalidArgument, "%s: padded N smaller than pad128(n)", name);
+  // SwiGLU: W holds a and g interleaved in 128-row blocks (np = 2 pad128(n)).
+  if (act == 2 && np != 2 * kp_out)
+    return set_error(kUnsupported,
+                     "%s: SwiGLU takes the interleaved [a | g] weight (padded N = 2 pad128(n))", name);
+  if (gemm_too_large(mp, np, kp, act == 2 || (mp >= 1024 && np >= 1024) ? 256 : 128))
+    return set_error(kUnsupported, "%s: problem too large for 32-bit tile offsets", name);
+  const GemmArgs g{static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(a_scales),
+                   static_cast<const uint8_t*>(w), static_cast<const uint8_t*>(w_scales), mp, np, kp,
+                   Epilogue{static_cast<const uint16_t*>(bias), nullptr, 0, nullptr, 0, nullptr, nullptr,
+                            0, nonfinite, n % 8 == 0 ? 1 : 0, static_cast<uint8_t*>(q),
+                            static_cast<uint8_t*>(scales), kp_out, act},
+                   out_rows, n};
+  return launch_gemm_planned(g, gemm_mode(g.ep), workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
 
 }  // namespace
 }  // namespace vdn
@@ -1114,39 +1102,19 @@ VDN_API int vdn_mxfp8_gemm(const void* a, const void* a_scales, int64_t mp, cons
                            const void* addend, int64_t ld_add, const void* residual,
                            int64_t ld_res, const void* gate, void* out, int64_t out_rows,
                            int64_t n, int64_t ldc, uint32_t* nonfinite, void* stream) {
-  const char* name = "vdn_mxfp8_gemm";
-  if (a == nullptr || a_scales == nullptr || w == nullptr || w_scales == nullptr || out == nullptr)
-    return set_error(kInvalidArgument, "%s: null pointer argument", name);
-  if (mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128)
-    return set_error(kInvalidArgument, "%s: padded M/N/K must be positive multiples of 128", name);
-  if (n <= 0 || n > np || out_rows < 0 || out_rows > mp || ldc < n ||
-      (addend != nullptr && ld_add < n) || (residual != nullptr && ld_res < n))
-    return set_error(kInvalidArgument, "%s: invalid output geometry", name);
-  if (gate != nullptr && residual == nullptr)
-    return set_error(kInvalidArgument, "%s: a gate needs a residual", name);
-  if (!aligned(a, 16) || !aligned(w, 16) || !aligned(a_scales, 4) || !aligned(w_scales, 4))
-    return set_error(kInvalidArgument, "%s: code buffers need 16-byte, scales 4-byte alignment",
-                     name);
-  if (out_rows == 0) return kOk;
-  auto st = static_cast<hipStream_t>(stream);
-  auto* ap = static_cast<const uint8_t*>(a);
-  auto* asp = static_cast<const uint8_t*>(a_scales);
-  auto* wp = static_cast<const uint8_t*>(w);
-  auto* wsp = static_cast<const uint8_t*>(w_scales);
-  const bool vec = n % 8 == 0 && ldc % 8 == 0 && aligned(out, 16) &&
-                   (bias == nullptr || aligned(bias, 16)) && (gate == nullptr || aligned(gate, 16)) &&
-                   (addend == nullptr || (ld_add % 8 == 0 && aligned(addend, 16))) &&
-                   (residual == nullptr || (ld_res % 8 == 0 && aligned(residual, 16)));
-  const Epilogue ep{static_cast<const uint16_t*>(bias), static_cast<const uint16_t*>(addend),
-                    ld_add, static_cast<const uint16_t*>(residual), ld_res,
-                    static_cast<const uint16_t*>(gate), static_cast<uint16_t*>(out), ldc,
-                    nonfinite, vec ? 1 : 0, nullptr, nullptr, 0, 0};
-  if (mp >= 1024 && np >= 1024) {
-    if (vec && addend == nullptr)
-      return launch_persistent(ap, asp, mp, wp, wsp, np, kp, ep, out_rows, n, st);
-    return launch_gemm<256, 256, 2, 2>(ap, asp, mp, wp, wsp, np, kp, ep, out_rows, n, st);
-  }
-  return launch_gemm<128, 128, 2, 2>(ap, asp, mp, wp, wsp, np, kp, ep, out_rows, n, st);
+  return gemm("vdn_mxfp8_gemm", a, a_scales, mp, w, w_scales, np, kp, bias, addend, ld_add, residual, ld_res,
+              gate, out, out_rows, n, ldc, nonfinite, nullptr, 0, stream);
+}
+
+VDN_API int vdn_mxfp8_gemm_ws(const void* a, const void* a_scales, int64_t mp, const void* w,
+                              const void* w_scales, int64_t np, int64_t kp, const void* bias,
+                              const void* addend, int64_t ld_add, const void* residual,
+                              int64_t ld_res, const void* gate, void* out, int64_t out_rows,
+                              int64_t n, int64_t ldc, uint32_t* nonfinite, void* workspace,
+                              int64_t workspace_bytes, void* stream) {
+  return gemm("vdn_mxfp8_gemm_ws", a, a_scales, mp, w, w_scales, np, kp, bias, addend, ld_add, residual,
+              ld_res, gate, out, out_rows, n, ldc, nonfinite, static_cast<float*>(workspace), workspace_bytes,
+              stream);
 }
 
 // Fused FFN producer: the GEMM of vdn_mxfp8_gemm (+ bias), then act (0 none, 1 GELU-tanh,
@@ -1163,38 +1131,26 @@ VDN_API int vdn_mxfp8_gemm_act_quantize(const void* a, const void* a_scales, int
                                         int64_t kp, const void* bias, int act, void* q,
                                         void* scales, int64_t out_rows, int64_t n,
                                         uint32_t* nonfinite, void* stream) {
-  const char* name = "vdn_mxfp8_gemm_act_quantize";
-  if (a == nullptr || a_scales == nullptr || w == nullptr || w_scales == nullptr || q == nullptr ||
-      scales == nullptr)
-    return set_error(kInvalidArgument, "%s: null pointer argument", name);
-  if (mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128)
-    return set_error(kInvalidArgument, "%s: padded M/N/K must be positive multiples of 128", name);
-  if (n <= 0 || n > np || out_rows < 0 || out_rows > mp)
-    return set_error(kInvalidArgument, "%s: invalid output geometry", name);
-  if (act != 0 && act != 1 && act != 2)
-    return set_error(kInvalidArgument, "%s: unknown activation %d", name, act);
-  if (!aligned(a, 16) || !aligned(w, 16) || !aligned(a_scales, 4) || !aligned(w_scales, 4) ||
-      !aligned(q, 16) || !aligned(scales, 4) || (bias != nullptr && !aligned(bias, 16)))
-    return set_error(kInvalidArgument, "%s: misaligned buffer", name);
-  if (out_rows == 0) return kOk;
-  const int64_t kp_out = (n + 127) / 128 * 128;
-  // Every column chunk up to kp_out must be produced: the padded GEMM width covers it.
-  if (kp_out > np) return set_error(kInvalidArgument, "%s: padded N smaller than pad128(n)", name);
-  // SwiGLU: W holds a and g interleaved in 128-row blocks (np = 2 pad128(n)); the hand-over
-  // between the a and g waves exists in the persistent kernel only.
-  if (act == 2 && (np != 2 * kp_out || mp < 1024 || np < 1024))
-    return set_error(kUnsupported,
-                     "%s: SwiGLU takes the interleaved [a | g] weight (padded N = 2 pad128(n)) "
-                     "and M >= 1024, N >= 512", name);
-  const Epilogue ep{static_cast<const uint16_t*>(bias), nullptr, 0, nullptr, 0, nullptr, nullptr,
-                    0, nonfinite, n % 8 == 0 ? 1 : 0, static_cast<uint8_t*>(q),
-                    static_cast<uint8_t*>(scales), kp_out, act};
-  auto st = static_cast<hipStream_t>(stream);
-  auto* ap = static_cast<const uint8_t*>(a);
-  auto* asp = static_cast<const uint8_t*>(a_scales);
-  auto* wp = static_cast<const uint8_t*>(w);
-  auto* wsp = static_cast<const uint8_t*>(w_scales);
-  if (mp >= 1024 && np >= 1024)
-    return launch_persistent(ap, asp, mp, wp, wsp, np, kp, ep, out_rows, n, st);
-  return launch_gemm<128, 128, 2, 2>(ap, asp, mp, wp, wsp, np, kp, ep, out_rows, n, st);
+  return gemm_act_quantize("vdn_mxfp8_gemm_act_quantize", a, a_scales, mp, w, w_scales, np, kp, bias, act, q,
+                           scales, out_rows, n, nonfinite, nullptr, 0, stream);
+}
+
+VDN_API int vdn_mxfp8_gemm_act_quantize_ws(const void* a, const void* a_scales, int64_t mp,
+                                           const void* w, const void* w_scales, int64_t np,
+                                           int64_t kp, const void* bias, int act, void* q,
+                                           void* scales, int64_t out_rows, int64_t n,
+                                           uint32_t* nonfinite, void* workspace,
+                                           int64_t workspace_bytes, void* stream) {
+  return gemm_act_quantize("vdn_mxfp8_gemm_act_quantize_ws", a, a_scales, mp, w, w_scales, np, kp, bias, act,
+                           q, scales, out_rows, n, nonfinite, static_cast<float*>(workspace), workspace_bytes,
+                           stream);
+}
+
+// kind: 0 bf16 output, 1 with a residual, 2 producer (no activation or GELU-tanh), 3 SwiGLU.
+VDN_API int vdn_mxfp8_gemm_workspace(int64_t mp, int64_t np, int64_t kp, int kind, int64_t* bytes) {
+  if (bytes == nullptr || mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128 || kind < 0 ||
+      kind > 3)
+    return set_error(kInvalidArgument, "vdn_mxfp8_gemm_workspace: invalid argument");
+  *bytes = gemm_workspace(mp, np, kp, kind);
+  return kOk;
 }
