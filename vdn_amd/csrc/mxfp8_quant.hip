@@ -233,7 +233,8 @@ __device__ __forceinline__ void unpack_bf16x8(const u32x4 w, float* f) {
 constexpr int kPrenormRows = 16;
 constexpr int kPrenormThreads = 64 * kPrenormRows;
 
-// Rows of exactly kCols = 512 kS columns (every slice real), eight rows per workgroup, two
+// Rows of exactly kCols = 512 kS (+ 256 with kHalf: a last slice in lanes 0 .. 31) columns, every
+// slice real, eight rows per workgroup, two
 // workgroups per CU (60 KB of LDS and at most 128 VGPRs each), so one's table staging and
 // load latency overlap the other's arithmetic; each wave issues its row's loads before the
 // table row is staged. The row index is wave-uniform, so every address is a scalar row base
@@ -242,11 +243,12 @@ constexpr int kPrenormThreads = 64 * kPrenormRows;
 // iff its magnitude bits reach 0x7f80, so one packed max per word tests two of them. (At
 // [108000, 5120]: 354 us without the bf16 output and 518 us with it, against 429 and 548 us
 // for sixteen rows per workgroup at one workgroup per CU, whose staging and arithmetic left
-// the CU without loads in flight.)
+// the CU without loads in flight. [4097, 5376], which the one-row workgroups of
+// prenorm_quantize_kernel took before, without the bf16 output: 82 -> 25 us.)
 constexpr int kFullRows = 8;
 constexpr int kFullThreads = 64 * kFullRows;
 
-template <int kS>
+template <int kS, bool kHalf>
 __global__ void __launch_bounds__(kFullThreads) __attribute__((amdgpu_waves_per_eu(4)))
 prenorm_quantize_full_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, int64_t stride,
                                   const void* __restrict__ weight, int weight_f32, float eps,
@@ -257,7 +259,8 @@ prenorm_quantize_full_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, 
                                   uint8_t* __restrict__ s, uint8_t* __restrict__ finite,
                                   int64_t rp) {
 #pragma clang fp contract(off)
-  constexpr int kCols = 64 * kS * 8;
+  constexpr int kCols = 512 * kS + (kHalf ? 256 : 0);
+  constexpr int kN = kS + (kHalf ? 1 : 0);   // 8-column slices of a lane
   constexpr int64_t kChunks = kCols / 128;
   __shared__ __attribute__((aligned(16))) float tab[3][kCols];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -268,14 +271,16 @@ prenorm_quantize_full_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, 
   const int64_t idx0 = r0 < rows ? indices[r0] : 0;
   int same = 1;
   if (tid < kFullRows && r0 + tid < rows) same = indices[r0 + tid] == idx0;
-  u32x4 raw[kS];
+  // slice j exists in this lane (the half slice fills whole 16-lane chunk groups)
+  auto has = [&](int j) { return j < kS || lane < 32; };
+  u32x4 raw[kN];
 #pragma unroll
-  for (int j = 0; j < kS; ++j) raw[j] = u32x4{0u, 0u, 0u, 0u};
+  for (int j = 0; j < kN; ++j) raw[j] = u32x4{0u, 0u, 0u, 0u};
   if (in_row) {
     const uint16_t* xrow = x + r * stride + lane * 8;
 #pragma unroll
-    for (int j = 0; j < kS; ++j)
-      raw[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(xrow + 512 * j));
+    for (int j = 0; j < kN; ++j)
+      if (has(j)) raw[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(xrow + 512 * j));
   }
   // one table row for the whole workgroup?
   const bool shared_row = __syncthreads_and(same) != 0;
@@ -305,7 +310,8 @@ prenorm_quantize_full_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, 
   const bool scale_lane = (lane & 15) == 0;
   if (!in_row) {  // a padding row: zero codes, the zero scale, finite
 #pragma unroll
-    for (int j = 0; j < kS; ++j) {
+    for (int j = 0; j < kN; ++j) {
+      if (!has(j)) continue;
       float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       quantize_store8_at(v, qlane + 512 * j, slane + 2048 * j, scale_lane);
     }
@@ -316,7 +322,7 @@ prenorm_quantize_full_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, 
   // sum of squares, two products per v_dot2 on the packed words, in two chains
   float ss0 = 0.f, ss1 = 0.f;
 #pragma unroll
-  for (int j = 0; j < kS; ++j) {
+  for (int j = 0; j < kN; ++j) {
     if (j & 1) ss1 = sumsq8_bf16(raw[j], ss1);
     else ss0 = sumsq8_bf16(raw[j], ss0);
   }
@@ -328,7 +334,8 @@ prenorm_quantize_full_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, 
   uint16_t* const ylane = y == nullptr ? nullptr : y + r * kCols + lane * 8;
   u16x2 mag = {0, 0};
 #pragma unroll
-  for (int j = 0; j < kS; ++j) {
+  for (int j = 0; j < kN; ++j) {
+    if (!has(j)) continue;
     const int c0 = (lane + 64 * j) * 8;
     float xv[8], w[8], u[8], sh[8];
     unpack_bf16x8(raw[j], xv);
@@ -691,22 +698,26 @@ VDN_API int vdn_mxfp8_prenorm_quantize(const void* x, int64_t rows, int64_t k, i
   const int64_t tab_align = tf ? 4 : 8;
   const bool wave_ok = vec && aligned16(weight) && aligned16(scale) && aligned16(shift) &&
                        scale_stride % tab_align == 0 && shift_stride % tab_align == 0;
-  if (wave_ok && slices <= 64 * 10) {
-    const dim3 grid(static_cast<unsigned>((rp + kPrenormRows - 1) / kPrenormRows));
-#define VDN_PRENORM_FULL(S)                                                                    \
-    if (k == 512 * (S)) {                                                                      \
-      hipLaunchKernelGGL((prenorm_quantize_full_rows_kernel<S>),                             \
+  if (wave_ok) {
+#define VDN_PRENORM_FULL(S, HALF)                                                              \
+    if (k == 512 * (S) + ((HALF) ? 256 : 0)) {                                                 \
+      hipLaunchKernelGGL((prenorm_quantize_full_rows_kernel<S, HALF>),                         \
                          dim3(static_cast<unsigned>((rp + kFullRows - 1) / kFullRows)),        \
                          dim3(kFullThreads), 0, st, xp, rows, row_stride, weight, wf, eps,     \
                          scale, scale_stride,                                                  \
                          shift, shift_stride, tf, indices, yp, qp, sp, finite, rp);            \
       return check_launch(name);                                                               \
     }
-    VDN_PRENORM_FULL(2)
-    VDN_PRENORM_FULL(4)
-    VDN_PRENORM_FULL(8)
-    VDN_PRENORM_FULL(10)
+    VDN_PRENORM_FULL(2, false)
+    VDN_PRENORM_FULL(3, false)
+    VDN_PRENORM_FULL(4, false)
+    VDN_PRENORM_FULL(8, false)
+    VDN_PRENORM_FULL(10, false)
+    VDN_PRENORM_FULL(10, true)
 #undef VDN_PRENORM_FULL
+  }
+  if (wave_ok && slices <= 64 * 10) {
+    const dim3 grid(static_cast<unsigned>((rp + kPrenormRows - 1) / kPrenormRows));
 #define VDN_PRENORM_WAVE(S)                                                                   \
     hipLaunchKernelGGL((prenorm_quantize_rows_kernel<S>), grid, dim3(kPrenormThreads), 0, st, xp, rows, \
                        k, row_stride, weight, wf, eps, scale, scale_stride, shift,              \
