@@ -248,7 +248,10 @@ constexpr int kPrenormThreads = 64 * kPrenormRows;
 constexpr int kFullRows = 8;
 constexpr int kFullThreads = 64 * kFullRows;
 
-template <int kS, bool kHalf>
+// kChains: how a row's sum of squares is ordered. 0: pairs on v_dot2 in two chains. 1 and 4 are the
+// orders of the kernels that took those widths before (one chain over a lane's slices; four, of
+// every fourth slice, each reduced over the wave), so their outputs stay the same bytes.
+template <int kS, bool kHalf, int kChains>
 __global__ void __launch_bounds__(kFullThreads) __attribute__((amdgpu_waves_per_eu(4)))
 prenorm_quantize_full_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, int64_t stride,
                                   const void* __restrict__ weight, int weight_f32, float eps,
@@ -319,16 +322,38 @@ prenorm_quantize_full_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, 
     return;
   }
   const int64_t table_row = shared_row ? idx0 : indices[r];
-  // sum of squares, two products per v_dot2 on the packed words, in two chains
-  float ss0 = 0.f, ss1 = 0.f;
+  float ss = 0.f;
+  if constexpr (kChains == 0) {
+    // two products per v_dot2 on the packed words, in two chains
+    float ss0 = 0.f, ss1 = 0.f;
 #pragma unroll
-  for (int j = 0; j < kN; ++j) {
-    if (j & 1) ss1 = sumsq8_bf16(raw[j], ss1);
-    else ss0 = sumsq8_bf16(raw[j], ss0);
+    for (int j = 0; j < kN; ++j) {
+      if (j & 1) ss1 = sumsq8_bf16(raw[j], ss1);
+      else ss0 = sumsq8_bf16(raw[j], ss0);
+    }
+    ss = ss0 + ss1;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+  } else {
+    float chain[kChains];
+#pragma unroll
+    for (int c = 0; c < kChains; ++c) {
+      chain[c] = 0.f;
+#pragma unroll
+      for (int j = c; j < kN; j += kChains) {
+        float f[8];
+        unpack_bf16x8(raw[j], f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) chain[c] += f[i] * f[i];
+      }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+      for (int c = 0; c < kChains; ++c) chain[c] += __shfl_xor(chain[c], off);
+#pragma unroll
+    for (int c = 0; c < kChains; ++c) ss += chain[c];
   }
-  float ss = ss0 + ss1;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
   const float ms = ss / static_cast<float>(kCols) + eps;
   const float inv_rms = static_cast<float>(1.0 / sqrt(static_cast<double>(ms)));
   uint16_t* const ylane = y == nullptr ? nullptr : y + r * kCols + lane * 8;
@@ -699,21 +724,21 @@ VDN_API int vdn_mxfp8_prenorm_quantize(const void* x, int64_t rows, int64_t k, i
   const bool wave_ok = vec && aligned16(weight) && aligned16(scale) && aligned16(shift) &&
                        scale_stride % tab_align == 0 && shift_stride % tab_align == 0;
   if (wave_ok) {
-#define VDN_PRENORM_FULL(S, HALF)                                                              \
+#define VDN_PRENORM_FULL(S, HALF, CHAINS)                                                            \
     if (k == 512 * (S) + ((HALF) ? 256 : 0)) {                                                 \
-      hipLaunchKernelGGL((prenorm_quantize_full_rows_kernel<S, HALF>),                         \
+      hipLaunchKernelGGL((prenorm_quantize_full_rows_kernel<S, HALF, CHAINS>),                 \
                          dim3(static_cast<unsigned>((rp + kFullRows - 1) / kFullRows)),        \
                          dim3(kFullThreads), 0, st, xp, rows, row_stride, weight, wf, eps,     \
                          scale, scale_stride,                                                  \
                          shift, shift_stride, tf, indices, yp, qp, sp, finite, rp);            \
       return check_launch(name);                                                               \
     }
-    VDN_PRENORM_FULL(2, false)
-    VDN_PRENORM_FULL(3, false)
-    VDN_PRENORM_FULL(4, false)
-    VDN_PRENORM_FULL(8, false)
-    VDN_PRENORM_FULL(10, false)
-    VDN_PRENORM_FULL(10, true)
+    VDN_PRENORM_FULL(2, false, 0)
+    VDN_PRENORM_FULL(3, false, 1)
+    VDN_PRENORM_FULL(4, false, 0)
+    VDN_PRENORM_FULL(8, false, 0)
+    VDN_PRENORM_FULL(10, false, 0)
+    VDN_PRENORM_FULL(10, true, 4)
 #undef VDN_PRENORM_FULL
   }
   if (wave_ok && slices <= 64 * 10) {
