@@ -25,6 +25,9 @@ int set_error(int status, const char* fmt, ...);
 // Checks the launch that was just queued on the current thread.
 int check_launch(const char* what);
 
+// Compute units of the current device (kept per device; mxfp8_gemm.hip).
+int cu_count();
+
 typedef __bf16 bf16;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));

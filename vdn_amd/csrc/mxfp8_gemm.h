@@ -90,7 +90,4 @@ int launch_gemm_planned(const GemmArgs& g, int mode, float* workspace, int64_t w
                         hipStream_t stream);
 int64_t gemm_workspace(int64_t mp, int64_t np, int64_t kp, int mode);
 
-// Compute units of the current device (cached per device).
-int cu_count();
-
 }  // namespace vdn
