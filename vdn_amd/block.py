@@ -327,10 +327,15 @@ class HybridDiTBlock(nn.Module):
         inner = cfg.inner
         frames, spatial = layout.num_frames, layout.tokens_per_frame
         dev = hidden.device
-        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = self.adaln_tables(temb)
-        idx = self._table_index(T, dev)
         parts = {} if return_parts else None
         nf = None if guard is None else torch.zeros(1, dtype=torch.int32, device=dev)
+        main = torch.cuda.current_stream(dev)
+        side = self._side_stream(dev) if (self.overlap_vda and parts is None) else None
+        if side is not None:
+            entered = torch.cuda.Event()
+            entered.record(main)
+        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = self.adaln_tables(temb)
+        idx = self._table_index(T, dev)
 
         def producer(finite):
             if guard is not None:
@@ -352,8 +357,6 @@ class HybridDiTBlock(nn.Module):
         raw_k = qkv[:, inner:2 * inner].view(T, heads, d)
         value = qkv[:, 2 * inner:].view(T, heads, d)
         cos, sin = rope
-        main = torch.cuda.current_stream(dev)
-        side = self._side_stream(dev) if (self.overlap_vda and parts is None) else None
 
         def gates(ready=None):
             soft_gate, beta, gate_down, partial = gate_projection(
@@ -376,11 +379,15 @@ class HybridDiTBlock(nn.Module):
             return vw.qk_rmsnorm(ck, k["norm_kc"], cfg.eps), cv
 
         if side is not None:
-            # The gate projection (x1 only) runs on the side stream beside the QK norm + RoPE
-            # pass; the window attention waits for its softmax gate through an event.
-            side.wait_stream(main)
+            # The context K and V of the cross-attention need only the caller's inputs: they run
+            # on the side stream beside the AdaLN, prenorm and QKV launches. The gate projection
+            # (x1 only) follows there beside the QK norm + RoPE pass; the window attention waits
+            # for its softmax gate through an event.
             gate_ready = torch.cuda.Event()
+            side.wait_event(entered)
             with torch.cuda.stream(side):
+                ck, cv = context_kv()
+                side.wait_stream(main)
                 soft_gate, beta, lin_gate, alpha = gates(gate_ready)
         else:
             soft_gate, beta, lin_gate, alpha = gates()
@@ -390,7 +397,7 @@ class HybridDiTBlock(nn.Module):
         # snapshots and quantized afterwards, which gives the same bytes.
         bounds = window_plan.bounds
         if parts is None:
-            qb, sb = mx.empty_activation(T, 2 * inner, dev)
+            qb, sb = mx.empty_activation(T, 2 * inner, dev, zero_padding=False)
 
             def linear_branch():
                 vv.vda_forward(raw_q, raw_k, value, beta, lin_gate, alpha, bounds,
@@ -399,10 +406,9 @@ class HybridDiTBlock(nn.Module):
 
             # The VDA branch runs on a side stream while RoPE and the window attention run on
             # the caller's stream (the reference's paper_vda_overlap, tensor_parallel.py:
-            # 202-216): its latency-bound passes fill the attention's gaps. The context K and V
-            # of the cross-attention follow it there. The tensors the side stream shares with
-            # the caller's stream (x1, qkv, the gates, alpha, the [O | O_lin] operand, the
-            # context K and V) are all released after main.wait_stream(side), so a later
+            # 202-216): its latency-bound passes fill the attention's gaps. The tensors the side
+            # stream shares with the caller's stream (x1, qkv, the gates, alpha, the [O | O_lin]
+            # operand, the context K and V) are all released after main.wait_stream(side), so a later
             # allocation on the caller's stream is ordered after the branch without
             # record_stream (which would keep ~5 GB per block out of the allocator's cache
             # while the host runs ahead); a side-stream allocation is ordered after them by
@@ -410,7 +416,6 @@ class HybridDiTBlock(nn.Module):
             if side is not None:
                 with torch.cuda.stream(side):
                     linear_branch()
-                    ck, cv = context_kv()
             q, kk = vw.paper_qk_rmsnorm_rope(raw_q, raw_k, k["norm_q"], k["norm_k"], cfg.eps,
                                              cos, sin, enabled=True)
             if side is not None:
@@ -454,7 +459,7 @@ class HybridDiTBlock(nn.Module):
             ck, cv = context_kv()
         if parts is None:
             # the queries' RMSNorm runs in the attention kernel as it loads them
-            qo, so = mx.empty_activation(T, inner, dev)
+            qo, so = mx.empty_activation(T, inner, dev, zero_padding=False)
             cross_attention(cq, ck, cv, cross_plan, d ** -0.5, out_mxfp8=(qo, so, 0),
                             q_norm=(k["norm_qc"], cfg.eps))
         else:

@@ -136,15 +136,16 @@ def _new_outputs(x: torch.Tensor, rows: int, k: int):
     return q, s, flag
 
 
-def empty_activation(rows: int, k: int, device):
+def empty_activation(rows: int, k: int, device, zero_padding: bool = True):
     """Codes [RP, KP] and flat swizzled scales for an MXFP8 activation that fused producers
     (vdn_window_attention_mxfp8, vdn_vda_readout_mxfp8) fill chunk by chunk. The padding rows
     rows .. RP-1 are zeroed here (codes 0, scale bytes 0), as the quantize producer leaves
-    them; every real row must then be written by the producers."""
+    them (zero_padding=False leaves them as they are, for an operand of a GEMM of `rows` rows only,
+    which stores nothing of the others); every real row must then be written by the producers."""
     rp, kp = padded_shape(rows, k)
     q = torch.empty((rp, kp), dtype=torch.uint8, device=device)
     s = torch.empty(scale_numel(rows, k), dtype=torch.uint8, device=device)
-    if rp > rows:
+    if zero_padding and rp > rows:
         q[rows:].zero_()
         # the scales of a 128-row block are one contiguous run of KP/128 x 512 bytes
         s[(rows // 128) * (kp // 128) * 512:].zero_()
