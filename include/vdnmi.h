@@ -192,6 +192,14 @@ int vdn_vda_scan(const float* CT, const float* CI, const float* seed, int chunks
                  int per_direction, float* bank, void* stream);
 
 /*
+ * vdn_vda_compose followed by vdn_vda_scan (per_direction = 1) in one pass over the frames, without
+ * the composed maps: bank [2, chunks, heads, 128, 128], chunk c covering frames starts[c] ..
+ * ends[c] - 1 (consecutive, from 0 to frames).
+ */
+int vdn_vda_chunk_scan(const float* T, const float* J, const float* seed, int frames, int heads,
+                       const int* starts, const int* ends, int chunks, float* bank, void* stream);
+
+/*
  * logp [frames + 1, heads, 128]: exclusive prefix sums of log(max(alpha, 1e-12)) over frames.
  * Replaces: the log-prefix of paper_gather (src/models/linear_attention/paper_stack.py:256).
  */

@@ -121,6 +121,34 @@ def test_scan_and_gather_fp64(device, frames, chunk, text, decay):
     assert bank.shape == (2, plan.chunks, h, 128, 128)
 
 
+@pytest.mark.parametrize("frames,heads,cuts_of,text", [(11, 48, (0, 4, 8, 11), True),
+                                                       (7, 72, (0, 1, 6, 7), False),
+                                                       (13, 40, (0, 5, 10, 13), True)])
+def test_chunk_scan_matches_fp64_and_composed_scan(device, frames, heads, cuts_of, text):
+    """One scan over the frames that stores the state at each chunk's far edge, against the float64
+    scan and against composing the chunks first (the same bank, in another fp32 order)."""
+    A, B, alpha = _stats(frames, heads, seed=heads)
+    t, inj = vv.paper_delta_factors(A.to(device), B.to(device), alpha.to(device))
+    seed = (torch.randn(heads, 128, 128) * .3).to(device) if text else None
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=device)
+    starts, ends, chunks = i32(cuts_of[:-1]), i32(cuts_of[1:]), len(cuts_of) - 1
+    bank, ct, ci, ref = (torch.full((2, chunks, heads, 128, 128), float("nan"), device=device)
+                         for _ in range(4))
+    st, sp = vv._stream(t), vv._lib.ptr(seed)
+    vv._lib.call("vdn_vda_chunk_scan", t.data_ptr(), inj.data_ptr(), sp, frames, heads,
+                 starts.data_ptr(), ends.data_ptr(), chunks, bank.data_ptr(), st)
+    vv._lib.call("vdn_vda_compose", t.data_ptr(), inj.data_ptr(), heads, starts.data_ptr(),
+                 ends.data_ptr(), chunks, ct.data_ptr(), ci.data_ptr(), st)
+    vv._lib.call("vdn_vda_scan", ct.data_ptr(), ci.data_ptr(), sp, chunks, heads, 1,
+                 ref.data_ptr(), st)
+    torch.testing.assert_close(bank, ref, atol=3e-6, rtol=3e-5)
+    prefix, suffix = ov.scan(t.cpu(), inj.cpu(), None if seed is None else seed.cpu())
+    torch.testing.assert_close(bank[0].double().cpu(), prefix[torch.tensor(cuts_of[1:]) - 1],
+                               atol=3e-6, rtol=3e-5)
+    torch.testing.assert_close(bank[1].double().cpu(), suffix[list(cuts_of[:-1])],
+                               atol=3e-6, rtol=3e-5)
+
+
 def test_gather_zero_decay_irregular_bounds_no_bridge(device):
     frames, h = 9, 1
     t = (torch.eye(128).expand(frames, h, 128, 128).contiguous() * .9)

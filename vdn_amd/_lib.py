@@ -45,6 +45,7 @@ SIGNATURES = {
     "vdn_vda_factors": [_ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr],
     "vdn_vda_compose": [_ptr, _ptr, _i32, _ptr, _ptr, _i32, _ptr, _ptr, _ptr],
     "vdn_vda_scan": [_ptr, _ptr, _ptr, _i32, _i32, _i32, _ptr, _ptr],
+    "vdn_vda_chunk_scan": [_ptr, _ptr, _ptr, _i32, _i32, _ptr, _ptr, _i32, _ptr, _ptr],
     "vdn_vda_log_prefix": [_ptr, _i32, _i32, _ptr, _ptr],
     "vdn_vda_gather": [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i32, _i32,
                        _i32, _i32, _ptr, _ptr],

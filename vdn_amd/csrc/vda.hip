@@ -489,7 +489,7 @@ vda_factors_kernel(const float* __restrict__ A, const float* __restrict__ B,
 // not depend on the state, so only the MFMA chain and the state exchange through LDS are
 // serial. With 8 KB of LDS and at most 96 VGPRs, five waves share a SIMD and every row
 // block, head and direction of a 40-head launch runs at once.
-enum RecurMode : int { kScan = 0, kCompose = 1 };
+enum RecurMode : int { kScan = 0, kCompose = 1, kChunkScan = 2 };
 
 constexpr int kRecWaves = 8;
 constexpr int kRecThreads = 64 * kRecWaves;
@@ -498,7 +498,7 @@ template <int kMode>
 __global__ void __launch_bounds__(kRecThreads) __attribute__((amdgpu_waves_per_eu(5)))
 vda_recur_kernel(const float* __restrict__ Tm, const float* __restrict__ Jm, int heads,
                  const int* __restrict__ starts, const int* __restrict__ ends, int chunks,
-                 const float* __restrict__ seed, int per_direction, float* __restrict__ out0,
+                 const float* __restrict__ seed, int per_direction, int frames, float* __restrict__ out0,
                  float* __restrict__ out1) {
   // state rows; compose keeps a second state (the accumulated injection b)
   __shared__ __attribute__((aligned(16))) float sS[kMode == kCompose ? 2 : 1][16 * 132];
@@ -507,13 +507,13 @@ vda_recur_kernel(const float* __restrict__ Tm, const float* __restrict__ Jm, int
   const int logical = xcd_contiguous(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
   const int rb = logical % (kD / 16);  // 16-row block
   const int ys = logical / (kD / 16);
-  const int ny = kMode == kScan ? heads : static_cast<int>(gridDim.x) / (kD / 16) / 2;
+  const int ny = kMode != kCompose ? heads : static_cast<int>(gridDim.x) / (kD / 16) / 2;
   const int by = ys % ny;
   const int dir = ys / ny;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r0 = rb * 16;
   int h, c = 0;
-  if (kMode == kScan) {
+  if (kMode != kCompose) {
     h = by;
   } else {
     h = by % heads;
@@ -522,15 +522,16 @@ vda_recur_kernel(const float* __restrict__ Tm, const float* __restrict__ Jm, int
   const int64_t mat = kD * kD;
   // number of frames in the sequence and the frame index of step t
   int n_steps, lo = 0, hi = 0;
-  if (kMode == kScan) {
-    n_steps = chunks;
+  const int scan_steps = kMode == kChunkScan ? frames : chunks;
+  if (kMode != kCompose) {
+    n_steps = scan_steps;
   } else {
     lo = starts[c];
     hi = ends[c];
     n_steps = hi - lo;
   }
   auto frame_of = [&](int t) {
-    if (kMode == kScan) return dir == 0 ? t : chunks - 1 - t;
+    if (kMode != kCompose) return dir == 0 ? t : scan_steps - 1 - t;
     return dir == 0 ? lo + t : hi - 1 - t;
   };
   // input matrix of frame/chunk x for head h: per-direction composed maps [2, C, H] or
@@ -546,7 +547,7 @@ vda_recur_kernel(const float* __restrict__ Tm, const float* __restrict__ Jm, int
   for (int idx = tid; idx < 16 * kD; idx += kRecThreads) {
     const int i = idx >> 7, j = idx & 127;
     float s0;
-    if (kMode == kScan) {
+    if (kMode != kCompose) {
       s0 = seed != nullptr ? seed[(static_cast<int64_t>(h) * kD + r0 + i) * kD + j] : 0.f;
     } else {
       s0 = (r0 + i) == j ? 1.f : 0.f;
@@ -579,8 +580,11 @@ vda_recur_kernel(const float* __restrict__ Tm, const float* __restrict__ Jm, int
   };
   if (n_steps > 0) load_step(0, tcur, jcur);
   __syncthreads();  // initial state written
+  int chunk = dir == 0 ? 0 : chunks - 1;   // kChunkScan: the chunk the scan is in
   for (int t = 0; t < n_steps; ++t) {
     const int x = frame_of(t);
+    // kChunkScan keeps the state at the chunk's far edge only
+    const bool edge = kMode == kChunkScan && (dir == 0 ? x + 1 == ends[chunk] : x == starts[chunk]);
     if (t + 1 < n_steps) load_step(t + 1, tnext, jnext);
     f32x4 acc[2];  // [state m / b]
 #pragma unroll
@@ -603,9 +607,11 @@ vda_recur_kernel(const float* __restrict__ Tm, const float* __restrict__ Jm, int
         float y = acc[a][v];
         if (a == inj) y += jcur[v];
         sS[a][i * 132 + j] = y;
-        if (kMode == kScan) out0[out_index(x) * mat + (r0 + i) * kD + j] = y;
+        if (kMode == kScan || edge)
+          out0[out_index(kMode == kScan ? x : chunk) * mat + (r0 + i) * kD + j] = y;
       }
     __syncthreads();  // the new state is complete
+    if (edge) chunk += dir == 0 ? (chunk + 1 < chunks ? 1 : 0) : (chunk > 0 ? -1 : 0);
 #pragma unroll
     for (int kk = 0; kk < kD / 4; ++kk) tcur[kk] = tnext[kk];
 #pragma unroll
@@ -1371,7 +1377,7 @@ VDN_API int vdn_vda_compose(const float* T, const float* J, int heads, const int
   const dim3 grid(kD / 16 * heads * chunks * 2);
   hipLaunchKernelGGL(vda_recur_kernel<kCompose>, grid, dim3(kRecThreads), 0,
                      static_cast<hipStream_t>(stream), T, J, heads, starts, ends, chunks,
-                     nullptr, 0, CT, CI);
+                     nullptr, 0, 0, CT, CI);
   return check_launch(name);
 }
 
@@ -1390,7 +1396,23 @@ VDN_API int vdn_vda_scan(const float* CT, const float* CI, const float* seed, in
   const dim3 grid(kD / 16 * heads * 2);
   hipLaunchKernelGGL(vda_recur_kernel<kScan>, grid, dim3(kRecThreads), 0,
                      static_cast<hipStream_t>(stream), CT, CI, heads, nullptr, nullptr, chunks,
-                     seed, per_direction, bank, nullptr);
+                     seed, per_direction, chunks, bank, nullptr);
+  return check_launch(name);
+}
+
+// vdn_vda_compose and vdn_vda_scan of the chunks in one pass over the frames: the scan runs through
+// the frame factors and stores its state at each chunk's far edge.
+VDN_API int vdn_vda_chunk_scan(const float* T, const float* J, const float* seed, int frames, int heads,
+                               const int* starts, const int* ends, int chunks, float* bank, void* stream) {
+  const char* name = "vdn_vda_chunk_scan";
+  if (T == nullptr || J == nullptr || starts == nullptr || ends == nullptr || bank == nullptr)
+    return set_error(kInvalidArgument, "%s: null pointer", name);
+  if (heads <= 0 || chunks <= 0 || frames < chunks) return set_error(kInvalidArgument, "%s: bad geometry", name);
+  if (static_cast<int64_t>(heads) * (kD / 16) * 2 > (1ll << 31) - 1)
+    return set_error(kUnsupported, "%s: grid too large", name);
+  hipLaunchKernelGGL(vda_recur_kernel<kChunkScan>, dim3(kD / 16 * heads * 2), dim3(kRecThreads), 0,
+                     static_cast<hipStream_t>(stream), T, J, heads, starts, ends, chunks, seed, 0, frames,
+                     bank, nullptr);
   return check_launch(name);
 }
 

@@ -315,6 +315,17 @@ def paper_boundary_plan(bounds, frames, device, chunk_size=8):
 
 # ----------------------------------------------------------------------- scan ----
 
+def _scan_frames(frames, heads, cuts):
+    """Whether one scan over all the frames beats composing the chunks and scanning those. The
+    scan's 16 x heads workgroups are all resident up to 64 heads and take about 6 us a frame; the
+    composition holds two states per chunk, about 10 us a frame, in waves of 1024 workgroups, and
+    then scans the chunks (56 heads, 35 frames in 7 chunks: 333 + 67 us against 252)."""
+    longest = max(b - a for a, b in zip(cuts[:-1], cuts[1:]))
+    chunks = len(cuts) - 1
+    waves = -(-16 * heads * chunks // 1024)
+    return 6 * frames * -(-heads // 64) < 10 * longest * waves + 6 * chunks
+
+
 def paper_boundary_scan(transitions, injections, plan, text_state=None):
     """Chunk composition, then both directional scans: bank [2, C, H, D, D] fp32
     (paper_stack.py:202-236). bank[0, c] is the forward state after chunk c; bank[1, c] the
@@ -346,6 +357,11 @@ def paper_boundary_scan(transitions, injections, plan, text_state=None):
         # every chunk is one frame: both directions scan the frame factors themselves
         _lib.call("vdn_vda_scan", transitions.data_ptr(), injections.data_ptr(),
                   _lib.ptr(text_state), plan.chunks, h, 0, bank.data_ptr(), stream)
+        return bank
+    if _scan_frames(f, h, plan.cuts):
+        _lib.call("vdn_vda_chunk_scan", transitions.data_ptr(), injections.data_ptr(),
+                  _lib.ptr(text_state), f, h, plan.starts.data_ptr(), plan.ends.data_ptr(),
+                  plan.chunks, bank.data_ptr(), stream)
         return bank
     ct = transitions.new_empty(shape)
     ci = transitions.new_empty(shape)
