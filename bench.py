@@ -698,8 +698,8 @@ def summarize_trace(stats_csv, bench_log, command):
             s_calls, s_ms = sum(c for c, _ in small), sum(t for _, t in small)
             out += ["The bench line times the family in the blocks without the side stream. In "
                     "the overlapped blocks the two context projections "
-                    "(`mxfp8_gemm_kernel<128, 128, ...>`) run on the side stream beside the "
-                    "window attention, whose workgroups hold the CUs, so their trace durations "
+                    "(`mxfp8_gemm_stream_kernel`) run on the side stream beside the AdaLN, "
+                    "prenorm and QKV launches, so their trace durations "
                     f"stretch (average {s_ms / s_calls:.4f} ms over {s_calls} launches). The "
                     "persistent kernel alone, the family's "
                     f"{100 * (g_ms - s_ms) / g_ms:.1f}% of GEMM time, averages "

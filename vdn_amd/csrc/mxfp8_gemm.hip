@@ -4,7 +4,11 @@
 // Replaces the reference's F.scaled_mm(BlockWise1x32, SWIZZLE_32_4_4) call in
 // MXFP8Linear.forward_quantized (src/models/ops/mxfp8_linear.py:61-93).
 //
-// Design:
+// Here: the general tile kernel (any epilogue operand and alignment), the persistent 256 x 256
+// kernel of large problems and the entry points. Small and middle sizes, and the choice by size:
+// mxfp8_gemm_stream.hip.
+//
+// Design of the general kernel:
 //   * one workgroup computes a BM x BN tile; its waves form a WGM x WGN grid and each
 //     wave owns a (BM/WGM) x (BN/WGN) sub-tile made of 16x16 outputs;
 //   * the inner product is v_mfma_scale_f32_16x16x128_f8f6f4. For 8-bit operands its K
