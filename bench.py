@@ -733,7 +733,7 @@ def _counter_rows(path, counter):
     return [(d, name, kib) for d, (name, kib) in per.items()]
 
 
-GEMM_KERNEL = re.compile(r"mxfp8_gemm_(persistent_)?kernel")
+GEMM_KERNEL = re.compile(r"mxfp8_gemm_((persistent|stream|finish)_)?kernel")
 
 
 def summarize_traffic(fetch_csv, write_csv, command=""):
