@@ -32,8 +32,7 @@ PEAK_HBM_GBS = 8000.0        # HBM3E, MI355X
 HEIGHT, WIDTH = 45, 80
 D = 128
 
-GEMMS = ("vdn_mxfp8_gemm", "vdn_mxfp8_gemm_act_quantize",
-         "vdn_mxfp8_gemm_ws", "vdn_mxfp8_gemm_act_quantize_ws")
+GEMMS = ("vdn_mxfp8_gemm", "vdn_mxfp8_gemm_act_quantize")
 VDA_ENTRIES = ("vdn_vda_statistics", "vdn_vda_factors", "vdn_vda_compose", "vdn_vda_scan",
                "vdn_vda_log_prefix", "vdn_vda_gather", "vdn_vda_readout", "vdn_vda_readout_mxfp8",
                "vdn_vda_readout_gated")
@@ -54,12 +53,12 @@ def padded(n):
 
 def work(name, a, plans):
     """Algorithmic (flop, bytes) of one launch from its C-ABI arguments."""
-    if name in ("vdn_mxfp8_gemm", "vdn_mxfp8_gemm_ws"):
+    if name == "vdn_mxfp8_gemm":
         kp, rows, n = a[6], a[14], a[15]
         ops = [a[7], a[8], a[10], a[12]]  # bias, addend, residual, gate
         extra = rows * n * 2 * sum(1 for p in ops[1:3] if p is not None)
         return 2.0 * rows * n * kp, rows * kp + n * kp + (rows + n) * kp / 32 + rows * n * 2 + extra
-    if name in ("vdn_mxfp8_gemm_act_quantize", "vdn_mxfp8_gemm_act_quantize_ws"):
+    if name == "vdn_mxfp8_gemm_act_quantize":
         kp, rows, n = a[6], a[11], a[12]
         kp_out = padded(n)
         return 2.0 * rows * n * kp, rows * kp + n * kp + (rows + n) * kp / 32 + rows * kp_out * (1 + 1 / 32)
@@ -733,7 +732,7 @@ def _counter_rows(path, counter):
     return [(d, name, kib) for d, (name, kib) in per.items()]
 
 
-GEMM_KERNEL = re.compile(r"mxfp8_gemm_((persistent|stream|finish)_)?kernel")
+GEMM_KERNEL = re.compile(r"mxfp8_gemm_((persistent|stream)_)?kernel")
 
 
 def summarize_traffic(fetch_csv, write_csv, command=""):
@@ -966,7 +965,7 @@ def main():
     inner = cfg.heads * cfg.head_dim
 
     def gemm_label(nm, a):
-        if nm in ("vdn_mxfp8_gemm_act_quantize", "vdn_mxfp8_gemm_act_quantize_ws"):
+        if nm == "vdn_mxfp8_gemm_act_quantize":
             return "ffn_up"
         kp, rows, n, res = a[6], a[14], a[15], a[10] is not None
         if rows != tokens:

@@ -99,12 +99,11 @@ int vdn_mxfp8_gemm_act_quantize(const void* a, const void* a_scales, int64_t mp,
                                 uint32_t* nonfinite, void* stream);
 
 /*
- * vdn_mxfp8_gemm and vdn_mxfp8_gemm_act_quantize with a caller's workspace (16-byte aligned,
- * private to the call until it has run on `stream`; contents immaterial). With at least the
- * bytes vdn_mxfp8_gemm_workspace reports, a problem with few tiles shares a tile's K steps
- * between workgroups, whose fp32 partials the workspace holds; with fewer (or null) it runs as
- * without. kind: 0 bf16 output, 1 with a residual, 2 producer (act 0 or 1), 3 SwiGLU (act 2);
- * 0 bytes: the problem has no use for a workspace.
+ * vdn_mxfp8_gemm and vdn_mxfp8_gemm_act_quantize with a caller's workspace (null, or 16-byte
+ * aligned), and the bytes of it that a problem uses: 0 at every size, so both forms run the same
+ * launches. Every output is summed over K in one sequence: a row's result does not depend on the
+ * number of rows, on the kernel its size takes or on a workspace. kind: 0 bf16 output, 1 with a
+ * residual, 2 producer (act 0 or 1), 3 SwiGLU (act 2).
  */
 int vdn_mxfp8_gemm_ws(const void* a, const void* a_scales, int64_t mp, const void* w,
                       const void* w_scales, int64_t np, int64_t kp, const void* bias,

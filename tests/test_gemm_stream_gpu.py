@@ -7,6 +7,8 @@ checked on sampled rows against the exactly dequantized float64 GEMM, within the
 bound of tests/test_mxfp8_gpu.py::test_gemm_gated_residual_epilogue, for the bf16, gated-residual
 and producer epilogues; without a workspace the same problem runs unshared.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -118,3 +120,73 @@ def test_stream_gemm_flags_nonfinite(device):
         flag.zero_()
         vm.mxfp8_gemm(q, s, wq, ws, n, rows=m - 1, nonfinite=flag)   # that row is no output now
         assert int(flag.item()) == 0
+
+
+def wide(rows, k, g):
+    """Normal values whose 32-column MXFP8 blocks lie up to 2^10 apart: their products' sums are far
+    from exact in fp32, so another order of them shows."""
+    scale = 2.0 ** torch.randint(-5, 6, (rows, k // 32, 1), generator=g)
+    return (torch.randn(rows, k // 32, 32, generator=g) * scale).reshape(rows, k).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("k", [256, 5120])
+def test_rows_do_not_depend_on_the_call(device, k):
+    """A row's output is the same bytes whatever number of rows the call has, and whichever kernels
+    that number takes: every kernel sums an output over K in one sequence. 1560 and 2177 rows leave
+    tiles over after whole rounds of the CUs; 77 and 300 have fewer tiles than CUs."""
+    n, rows = 5120, 3330
+    g = torch.Generator().manual_seed(k)
+    x = wide(rows, k, g).to(device)
+    wq, ws = vm.quantize_activation((wide(n, k, g) * 0.05).to(device))
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(device)
+    # the general tile kernel: rows of the output that 16-byte accesses do not cover
+    store = torch.empty(rows, n + 1, dtype=torch.bfloat16, device=device)
+    q, s = vm.quantize_activation(x)
+    ref = vm.mxfp8_gemm(q, s, wq, ws, n, rows=rows, bias=b, out=store[:, :n])
+    rq = vm.launch_quantize(ref.contiguous())[0]
+    for m in (1, 77, 300, 512, 960, 1560, 2177, rows):
+        q, s = vm.quantize_activation(x[:m])
+        got = vm.mxfp8_gemm(q, s, wq, ws, n, rows=m, bias=b)
+        assert torch.equal(got, ref[:m]), m
+        pq, _ = vm.mxfp8_gemm_act_quantize(q, s, wq, ws, n, rows=m, bias=b, act=None)
+        assert torch.equal(pq[:m], rq[:m]), m
+
+
+@pytest.mark.parametrize("m,n", [(77, 100), (77, 5119), (1560, 5119)])
+def test_producer_matches_separate_passes_at_odd_widths(device, m, n):
+    """A width that 16-byte accesses do not cover takes the general kernel for bf16 output and the
+    planned ones for the producer: the same bytes, also over many K steps."""
+    k = 5120
+    g = torch.Generator().manual_seed(m + n)
+    q, s = vm.quantize_activation(wide(m, k, g).to(device))
+    wq, ws = vm.quantize_activation((wide(n, k, g) * 0.05).to(device))
+    y = vm.mxfp8_gemm(q, s, wq, ws, n, rows=m)
+    for act, fn in ((None, vm.launch_quantize), ("gelu_tanh", vm.launch_gelu_quantize)):
+        fq, fs = vm.mxfp8_gemm_act_quantize(q, s, wq, ws, n, rows=m, act=act)
+        rq, rs = fn(y)[:2]
+        assert torch.equal(fq, rq) and torch.equal(fs, rs), act
+
+
+def test_workspace_forms_match(device):
+    """The entry points with a workspace run the same launches as those without."""
+    m, n, k = 77, 1280, 1152
+    g = torch.Generator().manual_seed(9)
+    q, s = vm.quantize_activation(wide(m, k, g).to(device))
+    wq, ws = vm.quantize_activation(wide(n, k, g).to(device))
+    size = ctypes.c_int64(-1)
+    _lib.call("vdn_mxfp8_gemm_workspace", q.shape[0], wq.shape[0], k, 0, ctypes.byref(size))
+    assert size.value == 0
+    work = torch.empty(1 << 20, dtype=torch.uint8, device=device)
+    ref = vm.mxfp8_gemm(q, s, wq, ws, n, rows=m)
+    rq, rs = vm.mxfp8_gemm_act_quantize(q, s, wq, ws, n, rows=m)
+    out, cq, cs = torch.zeros_like(ref), torch.zeros_like(rq), torch.zeros_like(rs)
+    head = (q.data_ptr(), s.data_ptr(), q.shape[0], wq.data_ptr(), ws.data_ptr(), wq.shape[0], k, None)
+    for space in ((work.data_ptr(), work.numel()), (None, 0)):
+        _lib.call("vdn_mxfp8_gemm_ws", *head, None, 0, None, 0, None, out.data_ptr(), m, n, n, None,
+                  *space, _lib.stream(device))
+        _lib.call("vdn_mxfp8_gemm_act_quantize_ws", *head, 1, cq.data_ptr(), cs.data_ptr(), m, n, None,
+                  *space, _lib.stream(device))
+        assert torch.equal(out, ref) and torch.equal(cq, rq) and torch.equal(cs, rs)
+    with pytest.raises(RuntimeError, match="alignment"):
+        _lib.call("vdn_mxfp8_gemm_ws", *head, None, 0, None, 0, None, out.data_ptr(), m, n, n, None,
+                  work.data_ptr() + 4, 1024, _lib.stream(device))

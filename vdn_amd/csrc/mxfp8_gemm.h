@@ -84,10 +84,7 @@ inline int gemm_mode(const Epilogue& ep) {
 // mxfp8_gemm.hip: the large-problem kernel (one workgroup per CU, 256 x 256 tiles).
 int launch_persistent(const GemmArgs& g, hipStream_t stream);
 
-// mxfp8_gemm_stream.hip: the large kernel, the stream kernel or both, by size. Without a
-// workspace no tile's K steps are shared between workgroups.
-int launch_gemm_planned(const GemmArgs& g, int mode, float* workspace, int64_t workspace_bytes,
-                        hipStream_t stream);
-int64_t gemm_workspace(int64_t mp, int64_t np, int64_t kp, int mode);
+// mxfp8_gemm_stream.hip: the large kernel, the stream kernel or both, by size.
+int launch_gemm_planned(const GemmArgs& g, int mode, hipStream_t stream);
 
 }  // namespace vdn

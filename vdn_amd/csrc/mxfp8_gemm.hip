@@ -1051,10 +1051,23 @@ int launch_gemm(const GemmArgs& g, hipStream_t stream) {
 
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
-int gemm(const char* name, const void* a, const void* a_scales, int64_t mp, const void* w,
-         const void* w_scales, int64_t np, int64_t kp, const void* bias, const void* addend, int64_t ld_add,
-         const void* residual, int64_t ld_res, const void* gate, void* out, int64_t out_rows, int64_t n,
-         int64_t ldc, uint32_t* nonfinite, float* workspace, int64_t workspace_bytes, void* stream) {
+}  // namespace
+}  // namespace vdn
+
+using namespace vdn;
+
+// Reference: src/models/ops/mxfp8_linear.py:61-93 (MXFP8Linear.forward_quantized: scaled_mm
+// BlockWise1x32 + SWIZZLE_32_4_4, crop to [rows, N], + bias in bf16), with the block's
+// following bf16 steps optionally fused into the epilogue: `addend` for
+// `out[video] += to_out_linear(...)` (hybrid_attention.py:254) and `residual`/`gate` for the
+// gated residual `hidden + gate * branch` (fused_block.py:49-51). `nonfinite` (nullable)
+// receives 1 when any stored output is not finite (mxfp8_linear.py:91-92).
+VDN_API int vdn_mxfp8_gemm(const void* a, const void* a_scales, int64_t mp, const void* w,
+                           const void* w_scales, int64_t np, int64_t kp, const void* bias,
+                           const void* addend, int64_t ld_add, const void* residual,
+                           int64_t ld_res, const void* gate, void* out, int64_t out_rows,
+                           int64_t n, int64_t ldc, uint32_t* nonfinite, void* stream) {
+  const char* name = "vdn_mxfp8_gemm";
   if (a == nullptr || a_scales == nullptr || w == nullptr || w_scales == nullptr || out == nullptr)
     return set_error(kInvalidArgument, "%s: null pointer argument", name);
   if (mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128)
@@ -1067,8 +1080,6 @@ int gemm(const char* name, const void* a, const void* a_scales, int64_t mp, cons
   if (!aligned(a, 16) || !aligned(w, 16) || !aligned(a_scales, 4) || !aligned(w_scales, 4))
     return set_error(kInvalidArgument, "%s: code buffers need 16-byte, scales 4-byte alignment",
                      name);
-  if (workspace != nullptr && (!aligned(workspace, 16) || workspace_bytes < 0))
-    return set_error(kInvalidArgument, "%s: the workspace needs 16-byte alignment", name);
   if (out_rows == 0) return kOk;
   const bool vec = n % 8 == 0 && ldc % 8 == 0 && aligned(out, 16) &&
                    (bias == nullptr || aligned(bias, 16)) && (gate == nullptr || aligned(gate, 16)) &&
@@ -1087,77 +1098,9 @@ int gemm(const char* name, const void* a, const void* a_scales, int64_t mp, cons
   auto st = static_cast<hipStream_t>(stream);
   // an addend, or rows that 16-byte accesses do not cover, take the general kernel
   if (vec && addend == nullptr)
-    return launch_gemm_planned(g, gemm_mode(g.ep), workspace, workspace_bytes, st);
+    return launch_gemm_planned(g, gemm_mode(g.ep), st);
   if (large) return launch_gemm<256, 256, 2, 2>(g, st);
   return launch_gemm<128, 128, 2, 2>(g, st);
-}
-
-int gemm_act_quantize(const char* name, const void* a, const void* a_scales, int64_t mp, const void* w,
-                      const void* w_scales, int64_t np, int64_t kp, const void* bias, int act, void* q,
-                      void* scales, int64_t out_rows, int64_t n, uint32_t* nonfinite, float* workspace,
-                      int64_t workspace_bytes, void* stream) {
-  if (a == nullptr || a_scales == nullptr || w == nullptr || w_scales == nullptr || q == nullptr ||
-      scales == nullptr)
-    return set_error(kInvalidArgument, "%s: null pointer argument", name);
-  if (mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128)
-    return set_error(kInvalidArgument, "%s: padded M/N/K must be positive multiples of 128", name);
-  if (n <= 0 || n > np || out_rows < 0 || out_rows > mp)
-    return set_error(kInvalidArgument, "%s: invalid output geometry", name);
-  if (act != 0 && act != 1 && act != 2)
-    return set_error(kInvalidArgument, "%s: unknown activation %d", name, act);
-  if (!aligned(a, 16) || !aligned(w, 16) || !aligned(a_scales, 4) || !aligned(w_scales, 4) ||
-      !aligned(q, 16) || !aligned(scales, 4) || (bias != nullptr && !aligned(bias, 16)))
-    return set_error(kInvalidArgument, "%s: misaligned buffer", name);
-  if (workspace != nullptr && (!aligned(workspace, 16) || workspace_bytes < 0))
-    return set_error(kInvalidArgument, "%s: the workspace needs 16-byte alignment", name);
-  if (out_rows == 0) return kOk;
-  const int64_t kp_out = (n + 127) / 128 * 128;
-  // Every column chunk up to kp_out must be produced: the padded GEMM width covers it.
-  if (kp_out > np) return set_error(kInvalidArgument, "%s: padded N smaller than pad128(n)", name);
-  // SwiGLU: W holds a and g interleaved in 128-row blocks (np = 2 pad128(n)).
-  if (act == 2 && np != 2 * kp_out)
-    return set_error(kUnsupported,
-                     "%s: SwiGLU takes the interleaved [a | g] weight (padded N = 2 pad128(n))", name);
-  if (gemm_too_large(mp, np, kp, act == 2 || (mp >= 1024 && np >= 1024) ? 256 : 128))
-    return set_error(kUnsupported, "%s: problem too large for 32-bit tile offsets", name);
-  const GemmArgs g{static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(a_scales),
-                   static_cast<const uint8_t*>(w), static_cast<const uint8_t*>(w_scales), mp, np, kp,
-                   Epilogue{static_cast<const uint16_t*>(bias), nullptr, 0, nullptr, 0, nullptr, nullptr,
-                            0, nonfinite, n % 8 == 0 ? 1 : 0, static_cast<uint8_t*>(q),
-                            static_cast<uint8_t*>(scales), kp_out, act},
-                   out_rows, n};
-  return launch_gemm_planned(g, gemm_mode(g.ep), workspace, workspace_bytes, static_cast<hipStream_t>(stream));
-}
-
-}  // namespace
-}  // namespace vdn
-
-using namespace vdn;
-
-// Reference: src/models/ops/mxfp8_linear.py:61-93 (MXFP8Linear.forward_quantized: scaled_mm
-// BlockWise1x32 + SWIZZLE_32_4_4, crop to [rows, N], + bias in bf16), with the block's
-// following bf16 steps optionally fused into the epilogue: `addend` for
-// `out[video] += to_out_linear(...)` (hybrid_attention.py:254) and `residual`/`gate` for the
-// gated residual `hidden + gate * branch` (fused_block.py:49-51). `nonfinite` (nullable)
-// receives 1 when any stored output is not finite (mxfp8_linear.py:91-92).
-VDN_API int vdn_mxfp8_gemm(const void* a, const void* a_scales, int64_t mp, const void* w,
-                           const void* w_scales, int64_t np, int64_t kp, const void* bias,
-                           const void* addend, int64_t ld_add, const void* residual,
-                           int64_t ld_res, const void* gate, void* out, int64_t out_rows,
-                           int64_t n, int64_t ldc, uint32_t* nonfinite, void* stream) {
-  return gemm("vdn_mxfp8_gemm", a, a_scales, mp, w, w_scales, np, kp, bias, addend, ld_add, residual, ld_res,
-              gate, out, out_rows, n, ldc, nonfinite, nullptr, 0, stream);
-}
-
-VDN_API int vdn_mxfp8_gemm_ws(const void* a, const void* a_scales, int64_t mp, const void* w,
-                              const void* w_scales, int64_t np, int64_t kp, const void* bias,
-                              const void* addend, int64_t ld_add, const void* residual,
-                              int64_t ld_res, const void* gate, void* out, int64_t out_rows,
-                              int64_t n, int64_t ldc, uint32_t* nonfinite, void* workspace,
-                              int64_t workspace_bytes, void* stream) {
-  return gemm("vdn_mxfp8_gemm_ws", a, a_scales, mp, w, w_scales, np, kp, bias, addend, ld_add, residual,
-              ld_res, gate, out, out_rows, n, ldc, nonfinite, static_cast<float*>(workspace), workspace_bytes,
-              stream);
 }
 
 // Fused FFN producer: the GEMM of vdn_mxfp8_gemm (+ bias), then act (0 none, 1 GELU-tanh,
@@ -1174,8 +1117,55 @@ VDN_API int vdn_mxfp8_gemm_act_quantize(const void* a, const void* a_scales, int
                                         int64_t kp, const void* bias, int act, void* q,
                                         void* scales, int64_t out_rows, int64_t n,
                                         uint32_t* nonfinite, void* stream) {
-  return gemm_act_quantize("vdn_mxfp8_gemm_act_quantize", a, a_scales, mp, w, w_scales, np, kp, bias, act, q,
-                           scales, out_rows, n, nonfinite, nullptr, 0, stream);
+  const char* name = "vdn_mxfp8_gemm_act_quantize";
+  if (a == nullptr || a_scales == nullptr || w == nullptr || w_scales == nullptr || q == nullptr ||
+      scales == nullptr)
+    return set_error(kInvalidArgument, "%s: null pointer argument", name);
+  if (mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128)
+    return set_error(kInvalidArgument, "%s: padded M/N/K must be positive multiples of 128", name);
+  if (n <= 0 || n > np || out_rows < 0 || out_rows > mp)
+    return set_error(kInvalidArgument, "%s: invalid output geometry", name);
+  if (act != 0 && act != 1 && act != 2)
+    return set_error(kInvalidArgument, "%s: unknown activation %d", name, act);
+  if (!aligned(a, 16) || !aligned(w, 16) || !aligned(a_scales, 4) || !aligned(w_scales, 4) ||
+      !aligned(q, 16) || !aligned(scales, 4) || (bias != nullptr && !aligned(bias, 16)))
+    return set_error(kInvalidArgument, "%s: misaligned buffer", name);
+  if (out_rows == 0) return kOk;
+  const int64_t kp_out = (n + 127) / 128 * 128;
+  // Every column chunk up to kp_out must be produced: the padded GEMM width covers it.
+  if (kp_out > np) return set_error(kInvalidArgument, "%s: padded N smaller than pad128(n)", name);
+  // SwiGLU: W holds a and g interleaved in 128-row blocks (np = 2 pad128(n)).
+  if (act == 2 && np != 2 * kp_out)
+    return set_error(kUnsupported,
+                     "%s: SwiGLU takes the interleaved [a | g] weight (padded N = 2 pad128(n))", name);
+  if (gemm_too_large(mp, np, kp, act == 2 || (mp >= 1024 && np >= 1024) ? 256 : 128))
+    return set_error(kUnsupported, "%s: problem too large for 32-bit tile offsets", name);
+  const GemmArgs g{static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(a_scales),
+                   static_cast<const uint8_t*>(w), static_cast<const uint8_t*>(w_scales), mp, np, kp,
+                   Epilogue{static_cast<const uint16_t*>(bias), nullptr, 0, nullptr, 0, nullptr, nullptr,
+                            0, nonfinite, n % 8 == 0 ? 1 : 0, static_cast<uint8_t*>(q),
+                            static_cast<uint8_t*>(scales), kp_out, act},
+                   out_rows, n};
+  return launch_gemm_planned(g, gemm_mode(g.ep), static_cast<hipStream_t>(stream));
+}
+
+// The forms with a caller's workspace, for programs built against them: no size uses one.
+static int check_workspace(const char* name, const void* workspace, int64_t bytes) {
+  if (workspace != nullptr && (!aligned(workspace, 16) || bytes < 0))
+    return set_error(kInvalidArgument, "%s: the workspace needs 16-byte alignment", name);
+  return kOk;
+}
+
+VDN_API int vdn_mxfp8_gemm_ws(const void* a, const void* a_scales, int64_t mp, const void* w,
+                              const void* w_scales, int64_t np, int64_t kp, const void* bias,
+                              const void* addend, int64_t ld_add, const void* residual,
+                              int64_t ld_res, const void* gate, void* out, int64_t out_rows,
+                              int64_t n, int64_t ldc, uint32_t* nonfinite, void* workspace,
+                              int64_t workspace_bytes, void* stream) {
+  const int status = check_workspace("vdn_mxfp8_gemm_ws", workspace, workspace_bytes);
+  if (status != kOk) return status;
+  return vdn_mxfp8_gemm(a, a_scales, mp, w, w_scales, np, kp, bias, addend, ld_add, residual, ld_res, gate,
+                        out, out_rows, n, ldc, nonfinite, stream);
 }
 
 VDN_API int vdn_mxfp8_gemm_act_quantize_ws(const void* a, const void* a_scales, int64_t mp,
@@ -1184,9 +1174,10 @@ VDN_API int vdn_mxfp8_gemm_act_quantize_ws(const void* a, const void* a_scales, 
                                            void* scales, int64_t out_rows, int64_t n,
                                            uint32_t* nonfinite, void* workspace,
                                            int64_t workspace_bytes, void* stream) {
-  return gemm_act_quantize("vdn_mxfp8_gemm_act_quantize_ws", a, a_scales, mp, w, w_scales, np, kp, bias, act,
-                           q, scales, out_rows, n, nonfinite, static_cast<float*>(workspace), workspace_bytes,
-                           stream);
+  const int status = check_workspace("vdn_mxfp8_gemm_act_quantize_ws", workspace, workspace_bytes);
+  if (status != kOk) return status;
+  return vdn_mxfp8_gemm_act_quantize(a, a_scales, mp, w, w_scales, np, kp, bias, act, q, scales, out_rows, n,
+                                     nonfinite, stream);
 }
 
 // kind: 0 bf16 output, 1 with a residual, 2 producer (no activation or GELU-tanh), 3 SwiGLU.
@@ -1194,6 +1185,6 @@ VDN_API int vdn_mxfp8_gemm_workspace(int64_t mp, int64_t np, int64_t kp, int kin
   if (bytes == nullptr || mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 || kp % 128 || kind < 0 ||
       kind > 3)
     return set_error(kInvalidArgument, "vdn_mxfp8_gemm_workspace: invalid argument");
-  *bytes = gemm_workspace(mp, np, kp, kind);
+  *bytes = 0;
   return kOk;
 }

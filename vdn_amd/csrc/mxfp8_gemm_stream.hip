@@ -12,9 +12,9 @@
 //            s % kSlots is free; the other MFMAs, with step s + kSlots's DMAs into that slot spread
 //            over them and each fragment register read again for step s + 1 after its last use.
 // Measured against the kernels it replaced at these sizes (us per launch, weights not in cache; M x
-// N x K): 77 x 5120 x 5120 51.6 -> 18, 512 x 5120 x 5120 49 -> 30, 960 x 5120 x 5120 66 -> 42,
-// 960 x 5120 x 13824 152 -> 97, 1560 x 5120 x 5120 65 -> 55, 1560 x 5120 x 13824 150 -> 113,
-// 2048 x 1536 x 6144 72 -> 28.
+// N x K): 77 x 5120 x 5120 48 -> 31, 512 x 5120 x 5120 49 -> 31, 960 x 5120 x 5120 68 -> 43,
+// 960 x 5120 x 13824 159 -> 98, 2048 x 1536 x 6144 67 -> 29; below 3072 rows of the large kernel
+// 3330 x 5376 x 14336 296 -> 222.
 #include "mxfp8_gemm.h"
 
 #include <algorithm>
@@ -80,16 +80,15 @@ __device__ __forceinline__ void stream_tile(int t, int tiles_m, int tiles_n, int
   tn = (t % in_band) / rows;
 }
 
-// How a launch's tiles fall on its workgroups: workgroup w first runs whole tiles w, w + grid, ..
-// (`whole` of them); then workgroup w < rest * parts runs part w % parts of the K steps of
-// remaining tile w / parts. With parts > 1 those tiles' fp32 partials are summed, in K order, by
-// the finishing kernel.
+// How a launch's tiles fall on its workgroups: workgroup w runs tiles w, w + grid, .. A tile's K
+// steps stay in one workgroup, in one sequence, as in the other GEMM kernels: shared between
+// workgroups, their partial sums would round differently, and a row's output would depend on how
+// many rows the call has and on the tile it falls in.
 struct StreamPlan {
   int bn, tiles_m, tiles_n;
   int grid;    // workgroups
-  int whole;   // whole tiles per workgroup
-  int rest;    // remaining tiles
-  int parts;   // K parts of a remaining tile (1: a whole tile too)
+  int rounds;  // tiles of every workgroup; the first `rest` have one more
+  int rest;
 };
 
 // ---- epilogue of a wave's 16-row group: kTN blocks of 16 columns, lane l holding rows l % 16,
@@ -314,7 +313,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 mxfp8_gemm_stream_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ As,
                          const uint8_t* __restrict__ W, const uint8_t* __restrict__ Ws, int64_t mp,
                          int64_t np, int64_t kp, Epilogue ep, int64_t out_rows, int64_t n,
-                         StreamPlan plan, float* __restrict__ partials) {
+                         StreamPlan plan) {
   constexpr int WGN = BN / 64, WGM = 4 / WGN;       // 4 waves: 1 x 4 (BN 256) or 2 x 2 (BN 128)
   constexpr int WM = kSM / WGM;
   constexpr int TM = WM / 16, TN = 4;
@@ -339,29 +338,7 @@ mxfp8_gemm_stream_kernel(const uint8_t* __restrict__ A, const uint8_t* __restric
   }
   const int nk = static_cast<int>(kp / kBK);
   const int64_t col_tiles = kp >> 7;
-  const int rest0 = plan.whole * grid;
-  const bool shares = w < plan.rest * plan.parts;
-
-  // ---- the workgroup's K steps as a sequence of segments (tile, first step, steps) ----
-  struct Cursor {
-    int i;                // segments taken
-    int tile, ks, left;   // current segment: next step and steps left (0: past the last segment)
-  };
-  auto next_segment = [&](Cursor& c) __attribute__((always_inline)) {
-    if (c.i < plan.whole) {
-      c.tile = w + c.i * grid;
-      c.ks = 0;
-      c.left = nk;
-    } else if (c.i == plan.whole && shares) {
-      const int part = w % plan.parts;
-      c.tile = rest0 + w / plan.parts;
-      c.ks = part * nk / plan.parts;
-      c.left = (part + 1) * nk / plan.parts - c.ks;
-    } else {
-      c.left = 0;
-    }
-    ++c.i;
-  };
+  const int tiles = plan.rounds + (w < plan.rest ? 1 : 0);   // of this workgroup
 
   // ---- DMA side ----
   // A wave loads rows kRowsA wave .. of the A tile and kRowsW wave .. of the W tile, 8 rows (1 KB)
@@ -382,19 +359,25 @@ mxfp8_gemm_stream_kernel(const uint8_t* __restrict__ A, const uint8_t* __restric
 #pragma unroll
   for (int i = 0; i < kSegW; ++i) voff_w[i] = lane_offset(wave * kRowsW + i * 8) - (i & 3) * 1024;
   const uint32_t voff_s = lane * 4;
-  Cursor d{0, 0, 0, 0};
+  struct Cursor {
+    int i;          // tiles taken
+    int ks, left;   // current tile: next K step and steps left (0: past the last tile)
+  };
+  Cursor d{0, 0, 0};
   Span d_a, d_w, d_s;
   // scale run of this wave: 0 the A block, 1 .. W's blocks (waves past the runs load one again)
   const int run = wave % kRuns;
   auto dma_tile = [&]() __attribute__((always_inline)) {
-    next_segment(d);
-    if (d.left == 0) {   // past the last step: empty resources, whose loads touch no memory
-      d.ks = 0;
+    d.ks = 0;
+    if (d.i >= tiles) {   // past the last tile: empty resources, whose loads touch no memory
+      d.left = 0;
       d_a = d_w = d_s = make_span(A, 0);
       return;
     }
     int tm, tn;
-    stream_tile(d.tile, plan.tiles_m, plan.tiles_n, tm, tn);
+    stream_tile(w + d.i * grid, plan.tiles_m, plan.tiles_n, tm, tn);
+    ++d.i;
+    d.left = nk;
     const int64_t dm0 = static_cast<int64_t>(tm) * kSM, dn0 = static_cast<int64_t>(tn) * BN;
     d_a = make_span(A + dm0 * kp, (mp - dm0) * kp);
     d_w = make_span(W + dn0 * kp, (np - dn0) * kp);
@@ -550,10 +533,8 @@ mxfp8_gemm_stream_kernel(const uint8_t* __restrict__ A, const uint8_t* __restric
       [&](auto i) __attribute__((always_inline)) { dma_one(kSlots - 1, i); });
 
   Epi epi(ep, lds + kSlots * kStep, lane, wave, wn, out_rows, n, mp);
-  Cursor c{0, 0, 0, 0};
-  next_segment(c);
-  for (; c.left != 0; next_segment(c)) {
-    // the segment's first step has landed for every wave (and so have the last epilogue's stores)
+  for (int t = 0; t < tiles; ++t) {
+    // the tile's first step has landed for every wave (and so have the last epilogue's stores)
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     {
       const uint8_t* buf = lds + slot * kStep;
@@ -573,34 +554,26 @@ mxfp8_gemm_stream_kernel(const uint8_t* __restrict__ A, const uint8_t* __restric
     for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
       for (int nt = 0; nt < TN; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int left = c.left; left > 0; --left) step();
-    if (c.left == nk) {
-      int tm, tn;
-      stream_tile(c.tile, plan.tiles_m, plan.tiles_n, tm, tn);
-      epi.begin_tile(static_cast<int64_t>(tm) * kSM, static_cast<int64_t>(tn) * BN);
-      epi.load_residual(wm * WM);
-      // one copy of the epilogue code: the accumulators are picked by a uniform branch chain
+    for (int left = nk; left > 0; --left) step();
+    int tm, tn;
+    stream_tile(w + t * grid, plan.tiles_m, plan.tiles_n, tm, tn);
+    epi.begin_tile(static_cast<int64_t>(tm) * kSM, static_cast<int64_t>(tn) * BN);
+    epi.load_residual(wm * WM);
+    // one copy of the epilogue code: the accumulators are picked by a uniform branch chain
 #pragma nounroll
-      for (int mt = 0; mt < TM; ++mt) {
-        f32x4 row[TN];
+    for (int mt = 0; mt < TM; ++mt) {
+      f32x4 row[TN];
 #pragma unroll
-        for (int m = 0; m < TM; ++m) {
-          if (m != mt) continue;
+      for (int m = 0; m < TM; ++m) {
+        if (m != mt) continue;
 #pragma unroll
-          for (int nt = 0; nt < TN; ++nt) {
-            row[nt] = acc[m][nt];
-            asm volatile("" : "+v"(row[nt]));   // opaque: stays in this branch
-          }
+        for (int nt = 0; nt < TN; ++nt) {
+          row[nt] = acc[m][nt];
+          asm volatile("" : "+v"(row[nt]));   // opaque: stays in this branch
         }
-        const int r = wm * WM + mt * 16;
-        epi.group(r, row, mt + 1 < TM ? r + 16 : -1);
       }
-    } else {
-      f32x4* dst = reinterpret_cast<f32x4*>(partials) + (static_cast<int64_t>(w) * 4 + wave) * (TM * TN * 64) + lane;
-#pragma unroll
-      for (int mt = 0; mt < TM; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < TN; ++nt) dst[(mt * TN + nt) * 64] = acc[mt][nt];
+      const int r = wm * WM + mt * 16;
+      epi.group(r, row, mt + 1 < TM ? r + 16 : -1);
     }
   }
   // DMAs past the last step must land before the workgroup's LDS is released
@@ -608,68 +581,36 @@ mxfp8_gemm_stream_kernel(const uint8_t* __restrict__ A, const uint8_t* __restric
   epi.finish();
 }
 
-// Sums the fp32 partials of the tiles whose K steps were shared, in step order, and finishes
-// them: one workgroup per remaining tile and 16-row group of each wave (many small workgroups:
-// the sums are bound by the latency of their loads).
-template <int BN, int kMode>
-__global__ void __launch_bounds__(256)
-mxfp8_gemm_finish_kernel(int64_t mp, Epilogue ep, int64_t out_rows, int64_t n, StreamPlan plan,
-                         const float* __restrict__ partials) {
-  constexpr int WGN = BN / 64, WGM = 4 / WGN, WM = kSM / WGM, TM = WM / 16, TN = 4;
-  using Epi = StreamEpilogue<BN, kMode>;
-  __shared__ __attribute__((aligned(16))) uint8_t strips[Epi::kStripBytes];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave / WGN, wn = wave % WGN;
-  const int q = blockIdx.x / TM, g = blockIdx.x % TM;
-  int tm, tn;
-  stream_tile(plan.whole * plan.grid + q, plan.tiles_m, plan.tiles_n, tm, tn);
-  Epi epi(ep, strips, lane, wave, wn, out_rows, n, mp);
-  epi.begin_tile(static_cast<int64_t>(tm) * kSM, static_cast<int64_t>(tn) * BN);
-  epi.load_residual(wm * WM + g * 16);
-  f32x4 acc[TN];
-#pragma unroll
-  for (int nt = 0; nt < TN; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const f32x4* src = reinterpret_cast<const f32x4*>(partials) +
-                     (static_cast<int64_t>(q) * plan.parts * 4 + wave) * (TM * TN * 64) + g * TN * 64 + lane;
-  for (int p = 0; p < plan.parts; ++p, src += 4 * TM * TN * 64)
-#pragma unroll
-    for (int nt = 0; nt < TN; ++nt) acc[nt] += src[nt * 64];
-  epi.group(wm * WM + g * 16, acc, -1);
-  epi.finish();
-}
-
 template <int BN, int kSlots, int kMode>
-void launch_stream_mode(const GemmArgs& g, const StreamPlan& p, float* partials, hipStream_t stream) {
+void launch_stream_mode(const GemmArgs& g, const StreamPlan& p, hipStream_t stream) {
   hipLaunchKernelGGL((mxfp8_gemm_stream_kernel<BN, kSlots, kMode>), dim3(p.grid), dim3(256), 0, stream, g.a,
-                     g.as, g.w, g.ws, g.mp, g.np, g.kp, g.ep, g.out_rows, g.n, p, partials);
-  if (p.parts > 1)
-    hipLaunchKernelGGL((mxfp8_gemm_finish_kernel<BN, kMode>), dim3(p.rest * (BN / 32)), dim3(256), 0, stream,
-                       g.mp, g.ep, g.out_rows, g.n, p, partials);
+                     g.as, g.w, g.ws, g.mp, g.np, g.kp, g.ep, g.out_rows, g.n, p);
 }
 
 template <int BN, int kSlots>
-int launch_stream(const GemmArgs& g, const StreamPlan& p, int mode, float* partials, hipStream_t stream) {
+int launch_stream(const GemmArgs& g, const StreamPlan& p, int mode, hipStream_t stream) {
   if (mode == 0)
-    launch_stream_mode<BN, kSlots, 0>(g, p, partials, stream);
+    launch_stream_mode<BN, kSlots, 0>(g, p, stream);
   else if (mode == 1)
-    launch_stream_mode<BN, kSlots, 1>(g, p, partials, stream);
+    launch_stream_mode<BN, kSlots, 1>(g, p, stream);
   else if (mode == 2)
-    launch_stream_mode<BN, kSlots, 2>(g, p, partials, stream);
+    launch_stream_mode<BN, kSlots, 2>(g, p, stream);
   else if constexpr (BN == 256)
-    launch_stream_mode<BN, kSlots, 3>(g, p, partials, stream);
+    launch_stream_mode<BN, kSlots, 3>(g, p, stream);
   return check_launch("vdn_mxfp8_gemm");
 }
 
-// ---- choice of the kernel and of the split, by estimated time ----
+// ---- choice of the kernel by estimated time ----
 // Microseconds, fitted to launches at M 77 .. 7395, N 1536 .. 21504, K 1536 .. 14336 on 256 CUs
-// with weights not in cache (estimates within about 15% of them):
+// with weights not in cache (estimates within 20% of launches of 25 us and more; the shorter ones,
+// all of the stream kernel, take as little as two thirds of theirs):
 //   large kernel    18 + per wave of 256 x 256 tiles 4 + 1.25 (1.32 over several waves) a K step
 //   stream, 256     10 + per 128 x 256 tile in sequence 3 + 0.80 (0.88) a K step
 //   stream, 128     10 + per 128 x 128 tile in sequence 2 + 0.47 (0.52) a K step
-// and for shared tiles a second launch and their fp32 partials, written and read back.
-// The plan depends on the padded sizes alone, not on the epilogue, so a projection and its fused
-// producer form sum every output in the same order and stay bit-identical.
+// Every kernel sums an output over K in one sequence, so the choice moves no bit of the result.
+// (Tiles left over after whole rounds with their K steps shared between workgroups: 1560 x 5120 x
+// 5120 55 us against 65, 77 x 5120 x 5120 18 against 31, but a row's bits then followed the row
+// count and the tile it fell in.)
 struct GemmPlan {
   int64_t large_rows;   // rows of the large kernel (a multiple of 256, or all); the rest: stream
   StreamPlan stream;
@@ -683,33 +624,23 @@ StreamPlan stream_plan(int64_t mp, int64_t np, int bn, int cus) {
   p.tiles_m = static_cast<int>(mp / kSM);
   p.tiles_n = static_cast<int>((np + bn - 1) / bn);
   const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
-  p.whole = static_cast<int>(tiles / cus);
+  p.rounds = static_cast<int>(tiles / cus);
   p.rest = static_cast<int>(tiles % cus);
-  p.parts = 1;
-  p.grid = p.whole > 0 ? cus : p.rest;
+  p.grid = p.rounds > 0 ? cus : p.rest;
   return p;
 }
 
-double best_stream(int64_t mp, int64_t np, int nk, bool may_split, int cus, StreamPlan* best) {
+double best_stream(int64_t mp, int64_t np, int nk, int cus, StreamPlan* best) {
   double best_cost = 1e30;
   for (int bn = 256; bn >= 128; bn -= 128) {
     if (bn * static_cast<int64_t>(nk) * kBK >= (1ll << 31)) continue;   // 32-bit offsets in a tile
-    StreamPlan p = stream_plan(mp, np, bn, cus);
+    const StreamPlan p = stream_plan(mp, np, bn, cus);
     const double tile = bn == 256 ? 3 : 2;
-    const double step = bn == 256 ? (p.whole > 0 ? 0.88 : 0.80) : (p.whole > 0 ? 0.52 : 0.47);
-    // Every remaining tile in the same number of parts of at least 4 steps. With whole tiles
-    // beside them only in 256-column tiles, which every epilogue has.
-    const int most = may_split && p.rest > 0 && (bn == 256 || p.whole == 0) ? std::min(cus / p.rest, 8) : 1;
-    for (int parts = 1; parts <= most && (parts == 1 || nk / parts >= 4); ++parts) {
-      p.parts = parts;
-      p.grid = p.whole > 0 ? cus : p.rest * parts;
-      double cost = 10 + p.whole * (nk * step + tile);
-      if (p.rest > 0) cost += (nk + parts - 1) / parts * step + tile;
-      if (parts > 1) cost += 5 + p.rest * parts * (kSM * bn * 8) / 10e6;   // 4 + 4 bytes at about 10 TB/s (cached)
-      if (cost < best_cost) {
-        best_cost = cost;
-        *best = p;
-      }
+    const double step = bn == 256 ? (p.rounds > 0 ? 0.88 : 0.80) : (p.rounds > 0 ? 0.52 : 0.47);
+    const double cost = 10 + (p.rounds + (p.rest > 0 ? 1 : 0)) * (nk * step + tile);
+    if (cost < best_cost) {
+      best_cost = cost;
+      *best = p;
     }
   }
   return best_cost;
@@ -718,17 +649,17 @@ double best_stream(int64_t mp, int64_t np, int nk, bool may_split, int cus, Stre
 // The large kernel wins once its tiles fill the CUs for whole waves (its step moves half the
 // bytes per FLOP); what is left over, and small problems, run faster in the stream kernel's
 // smaller tiles. 5% in the estimate decides for one launch of the large kernel.
-GemmPlan plan_gemm(int64_t mp, int64_t np, int64_t kp, int mode, bool may_split) {
+GemmPlan plan_gemm(int64_t mp, int64_t np, int64_t kp, int mode) {
   const int cus = cu_count(), nk = static_cast<int>(kp / kBK);
   GemmPlan plan{0, {}};
-  double best = best_stream(mp, np, nk, may_split, cus, &plan.stream);
+  double best = best_stream(mp, np, nk, cus, &plan.stream);
   if (mp >= 1024 && np >= 1024) {
     const int64_t tiles_m = (mp + 255) / 256, tiles_n = (np + 255) / 256, tiles = tiles_m * tiles_n;
     const int64_t waves = tiles / cus, rows = waves * cus / tiles_n;
     if (waves > 0 && rows > 0 && rows < tiles_m) {
       StreamPlan rest;
       const double both = large_cost((rows * tiles_n + cus - 1) / cus, nk) +
-                          best_stream(mp - rows * 256, np, nk, may_split, cus, &rest);
+                          best_stream(mp - rows * 256, np, nk, cus, &rest);
       if (both < best) {
         best = both;
         plan.large_rows = rows * 256;
@@ -737,31 +668,15 @@ GemmPlan plan_gemm(int64_t mp, int64_t np, int64_t kp, int mode, bool may_split)
     }
     if (best >= 0.95 * large_cost((tiles + cus - 1) / cus, nk)) plan.large_rows = mp;
   }
-  // SwiGLU's halves meet in a 256-column tile: the same parts in those
-  if (mode == 3 && plan.stream.bn == 128) {
-    const int parts = plan.stream.parts;
-    plan.stream = stream_plan(mp - plan.large_rows, np, 256, cus);
-    plan.stream.parts = parts;
-    if (plan.stream.whole == 0) plan.stream.grid = plan.stream.rest * parts;
-  }
+  // SwiGLU's halves meet in a 256-column tile
+  if (mode == 3 && plan.stream.bn == 128) plan.stream = stream_plan(mp - plan.large_rows, np, 256, cus);
   return plan;
-}
-
-int64_t plan_workspace(const GemmPlan& plan, int64_t mp) {
-  if (plan.large_rows >= mp || plan.stream.parts == 1) return 0;
-  return static_cast<int64_t>(plan.stream.rest) * plan.stream.parts * kSM * plan.stream.bn * 4;
 }
 
 }  // namespace
 
-int64_t gemm_workspace(int64_t mp, int64_t np, int64_t kp, int mode) {
-  return plan_workspace(plan_gemm(mp, np, kp, mode, true), mp);
-}
-
-int launch_gemm_planned(const GemmArgs& g, int mode, float* workspace, int64_t workspace_bytes,
-                        hipStream_t stream) {
-  GemmPlan plan = plan_gemm(g.mp, g.np, g.kp, mode, workspace != nullptr);
-  if (plan_workspace(plan, g.mp) > workspace_bytes) plan = plan_gemm(g.mp, g.np, g.kp, mode, false);
+int launch_gemm_planned(const GemmArgs& g, int mode, hipStream_t stream) {
+  const GemmPlan plan = plan_gemm(g.mp, g.np, g.kp, mode);
   if (plan.large_rows > 0) {
     GemmArgs top = g;
     if (plan.large_rows < g.mp) {
@@ -786,8 +701,8 @@ int launch_gemm_planned(const GemmArgs& g, int mode, float* workspace, int64_t w
     low.ep.q_out += r * g.ep.kp_out;
     low.ep.s_out += r / 128 * (g.ep.kp_out / 128) * 512;
   }
-  return plan.stream.bn == 256 ? launch_stream<256, 3>(low, plan.stream, mode, workspace, stream)
-                               : launch_stream<128, 4>(low, plan.stream, mode, workspace, stream);
+  return plan.stream.bn == 256 ? launch_stream<256, 3>(low, plan.stream, mode, stream)
+                               : launch_stream<128, 4>(low, plan.stream, mode, stream);
 }
 
 }  // namespace vdn

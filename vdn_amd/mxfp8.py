@@ -7,8 +7,6 @@ Triton, no scaled_mm and no fallback: a device or build problem raises RuntimeEr
 """
 from __future__ import annotations
 
-import ctypes
-import functools
 import math
 
 import numpy as np
@@ -341,24 +339,6 @@ def _nonfinite_flag(nonfinite, check_finite, device):
     return torch.zeros(1, dtype=torch.int32, device=device) if check_finite else None
 
 
-@functools.lru_cache(maxsize=4096)
-def _workspace_bytes(mp, np_, kp, kind):
-    size = ctypes.c_int64(0)
-    _lib.call("vdn_mxfp8_gemm_workspace", mp, np_, kp, kind, ctypes.byref(size))
-    return size.value
-
-
-def _call_gemm(name, mp, np_, kp, kind, device, *args):
-    """Entry point `name`, or its _ws form with a workspace from the caching allocator (whose
-    reuse is ordered on the current stream) where the problem shares tiles between workgroups."""
-    size = _workspace_bytes(mp, np_, kp, kind)
-    if size:
-        work = torch.empty(size, dtype=torch.uint8, device=device)
-        _lib.call(name + "_ws", *args, work.data_ptr(), size, _lib.stream(device))
-    else:
-        _lib.call(name, *args, _lib.stream(device))
-
-
 def mxfp8_gemm(data, scales, weight_data, weight_scale, n, *, rows=None, bias=None, out=None,
                accumulate=False, addend=None, residual=None, gate=None, check_finite=False,
                nonfinite=None):
@@ -416,11 +396,10 @@ def mxfp8_gemm(data, scales, weight_data, weight_scale, n, *, rows=None, bias=No
     _check_alias(out, residual, rows, n, "residual")
     flag = _nonfinite_flag(nonfinite, check_finite, dev)
     if rows:
-        _call_gemm("vdn_mxfp8_gemm", mp, np_, kp, 0 if residual is None else 1, dev,
-                   data.data_ptr(), scales.data_ptr(), mp, weight_data.data_ptr(),
-                   weight_scale.data_ptr(), np_, kp, _lib.ptr(bias), add_ptr, ld_add, res_ptr, ld_res,
-                   _lib.ptr(gate), out.data_ptr(), rows, n, out.stride(0) if rows > 1 else n,
-                   _lib.ptr(flag))
+        _lib.call("vdn_mxfp8_gemm", data.data_ptr(), scales.data_ptr(), mp,
+                  weight_data.data_ptr(), weight_scale.data_ptr(), np_, kp, _lib.ptr(bias),
+                  add_ptr, ld_add, res_ptr, ld_res, _lib.ptr(gate), out.data_ptr(), rows, n,
+                  out.stride(0) if rows > 1 else n, _lib.ptr(flag), _lib.stream(data.device))
     if check_finite and int(flag.item()) != 0:
         raise ValueError("nonfinite MXFP8 result")
     return out
@@ -457,10 +436,9 @@ def _gemm_swiglu_quantize(data, scales, weight_data, weight_scale, n, rows, bias
     s = torch.empty(mp * kp_out // 32, dtype=torch.uint8, device=data.device)
     flag = _nonfinite_flag(nonfinite, check_finite, data.device)
     if rows:
-        _call_gemm("vdn_mxfp8_gemm_act_quantize", mp, np_, kp, 3, data.device,
-                   data.data_ptr(), scales.data_ptr(), mp, weight_data.data_ptr(),
-                   weight_scale.data_ptr(), np_, kp, _lib.ptr(bias), 2, q.data_ptr(), s.data_ptr(),
-                   rows, n, _lib.ptr(flag))
+        _lib.call("vdn_mxfp8_gemm_act_quantize", data.data_ptr(), scales.data_ptr(), mp,
+                  weight_data.data_ptr(), weight_scale.data_ptr(), np_, kp, _lib.ptr(bias), 2,
+                  q.data_ptr(), s.data_ptr(), rows, n, _lib.ptr(flag), _lib.stream(data.device))
     else:
         q.zero_()
         s.zero_()
@@ -473,7 +451,7 @@ def mxfp8_gemm_act_quantize(data, scales, weight_data, weight_scale, n, *, rows=
                             act="gelu_tanh", check_finite=False, nonfinite=None):
     """MXFP8 codes/scales of act(bf16(dequant(data) @ dequant(weight)ᵀ + bias)) for the next
     projection, produced in the GEMM epilogue. Bit-identical to mxfp8_gemm over the same weight
-    (both sum K in the same order at every size) followed by
+    (both sum K in one sequence at every size and width) followed by
     launch_gelu_quantize (act "gelu_tanh"), launch_quantize (act None) or, for act "swiglu"
     over a weight from interleave_swiglu (n = the SwiGLU width), launch_swiglu_quantize of
     the [a | g] output. `nonfinite` (int32 [1] on the device) becomes nonzero on an inf/NaN
@@ -494,10 +472,10 @@ def mxfp8_gemm_act_quantize(data, scales, weight_data, weight_scale, n, *, rows=
     s = torch.empty(mp * kp_out // 32, dtype=torch.uint8, device=data.device)
     flag = _nonfinite_flag(nonfinite, check_finite, data.device)
     if rows:
-        _call_gemm("vdn_mxfp8_gemm_act_quantize", mp, np_, kp, 2, data.device,
-                   data.data_ptr(), scales.data_ptr(), mp, weight_data.data_ptr(),
-                   weight_scale.data_ptr(), np_, kp, _lib.ptr(bias), 1 if act == "gelu_tanh" else 0,
-                   q.data_ptr(), s.data_ptr(), rows, n, _lib.ptr(flag))
+        _lib.call("vdn_mxfp8_gemm_act_quantize", data.data_ptr(), scales.data_ptr(), mp,
+                  weight_data.data_ptr(), weight_scale.data_ptr(), np_, kp, _lib.ptr(bias),
+                  1 if act == "gelu_tanh" else 0, q.data_ptr(), s.data_ptr(), rows, n,
+                  _lib.ptr(flag), _lib.stream(data.device))
     else:
         q.zero_()
         s.zero_()
