@@ -129,6 +129,53 @@ def test_gate_projection_matches_oracle(wide, odd, frames, spatial, width):
     np.testing.assert_allclose(alpha.double().numpy(), expect.numpy(), rtol=2e-5, atol=1e-7)
 
 
+@pytest.mark.parametrize("frames,spatial", [(13, 300), (9, 1000)])
+def test_gate_projection_of_more_row_blocks_matches_oracle(wide, frames, spatial):
+    """39 and 72 row blocks, each frame's last one partial. The gates within one bf16 rounding of the
+    float64 oracle. Among this many down values some cancel to where an fp32 ulp of the addends
+    exceeds a bf16 ulp of the sum: K 2^-24 of the addends' magnitudes (any order of an fp32 sum)
+    is allowed beside the rounding; nearly all are equal."""
+    g = torch.Generator().manual_seed(frames)
+    x1 = torch.randn(frames * spatial, WIDE.hidden, generator=g).to(torch.bfloat16).double()
+    soft, beta, _, down, partial = kernel_gates(wide.tensors, WIDE, x1, frames)
+    o_soft, o_beta, _ = ob.BlockOracle(wide.tensors, WIDE).small_projections(x1)
+    for name, a, ref in (("soft", soft, o_soft), ("beta", beta, o_beta)):
+        u = _ulps(a, ref)
+        assert u.max() <= 1.0, (name, u.max())
+        assert (u == 0).mean() >= 0.97, (name, (u == 0).mean())
+    wd = wide.lgate_down_w.double()
+    ref, mag = x1 @ wd.T, x1.abs() @ wd.abs().T
+    limit = torch.from_numpy(omx.bf16_ulp(ref.numpy())) + WIDE.hidden * 2.0 ** -24 * mag
+    assert bool(((down - ref).abs() <= limit).all())
+    assert (_ulps(down, _bf16(ref.numpy())) == 0).mean() >= 0.97
+    bpf = -(-spatial // 128)
+    sums = partial.double().view(frames, bpf, 128)
+    rows = (x1 @ wide.alpha_down_w.double().T).view(frames, spatial, 128)
+    for b in range(bpf):
+        np.testing.assert_allclose(sums[:, b].numpy(), rows[:, 128 * b:128 * b + 128].sum(1).numpy(),
+                                   rtol=1e-5, atol=1e-4)
+
+
+def test_gate_projection_is_the_same_bits_for_any_number_of_row_blocks(wide):
+    """Up to CUs / 12 row blocks of 128 run in twelve column groups, up to CUs / 4 in four, more in
+    one: frames computed in calls of each size give the same bytes, their last blocks partial. The
+    columns of x1 lie up to 2^10 apart, so another order of the fp32 sums would show."""
+    cfg, t = WIDE, _cuda(wide.tensors)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    spatial = 200                                    # two blocks a frame
+    counts = (cus // 24, cus // 24 + 1, cus // 8, cus // 8 + 1)
+    g = torch.Generator().manual_seed(21)
+    x1 = torch.randn(counts[-1] * spatial, cfg.hidden, generator=g)
+    x1 = (x1 * 2.0 ** torch.randint(-5, 6, (1, cfg.hidden), generator=g)).to(torch.bfloat16).cuda()
+    w = vb.gate_weight(BlockWeights(t), cfg)
+    full = vb.gate_projection(x1, w, t["soft_gate_b"], cfg.heads, counts[-1], spatial)
+    assert 2 * counts[-1] * 4 > cus >= 2 * counts[2] * 4 and 2 * counts[0] * 12 <= cus < 2 * counts[1] * 12
+    for frames in counts[:-1]:
+        part = vb.gate_projection(x1[:frames * spatial], w, t["soft_gate_b"], cfg.heads, frames, spatial)
+        for name, a, b in zip(("soft gate", "beta", "down", "partial"), part, full):
+            assert torch.equal(a.reshape(-1), b.reshape(-1)[:a.numel()]), (frames, name)
+
+
 @pytest.mark.parametrize("hidden,m,dtype", [(512, 1, torch.float32), (5120, 1, torch.float32),
                                             (520, 3, torch.float32), (512, 2, torch.bfloat16),
                                             (512, 2, torch.float16)])
