@@ -85,7 +85,8 @@ int vdn_mxfp8_gemm(const void* a, const void* a_scales, int64_t mp, const void* 
 
 /*
  * Block-scaled GEMM feeding the next MXFP8 projection directly: y = bf16(bf16(acc) + bias),
- * act = 1 applies GELU-tanh (rounded to bf16; act = 0: none), and y is stored as MXFP8 codes
+ * act = 1 applies GELU-tanh (rounded to bf16; act = 0: none; act = 2: SwiGLU a * silu(g), over a
+ * weight with a and g interleaved in 128-row blocks, np = 2 pad128(n)), and y is stored as MXFP8 codes
  * q [mp, pad128(n)] + swizzled scales (mp * pad128(n) / 32 bytes), exactly what
  * vdn_mxfp8_act_quantize / vdn_mxfp8_quantize write for that bf16 matrix. Rows >= out_rows
  * and columns >= n are zero. *nonfinite (nullable) becomes 1 on a nonfinite activation.
@@ -116,6 +117,14 @@ int vdn_mxfp8_gemm_act_quantize_ws(const void* a, const void* a_scales, int64_t 
                                    uint32_t* nonfinite, void* workspace, int64_t workspace_bytes,
                                    void* stream);
 int vdn_mxfp8_gemm_workspace(int64_t mp, int64_t np, int64_t kp, int kind, int64_t* bytes);
+
+/*
+ * Which kernels run a problem of that size (kind as above) on the current device, for 16-byte
+ * accessible operands without an addend: large_rows rows from the first on in 256 x 256 tiles, the
+ * rows below (if any) in tiles of 128 x tile_cols (128 or 256; 0: there are none).
+ */
+int vdn_mxfp8_gemm_plan(int64_t mp, int64_t np, int64_t kp, int kind, int64_t* large_rows,
+                        int* tile_cols);
 
 /* ---------------------------------------------------------------------------------------
  * VDA linear-attention branch (D = 128). A 4-D operand "(f, h, s, c)" is addressed as

@@ -46,6 +46,11 @@ def test_invalid_arguments_are_rejected_without_a_device():
     assert lib.vdn_mxfp8_gemm(None, None, 128, None, None, 128, 128, None, None, 0, None, 0,
                               None, None, 1, 1, 1, None, None) != 0
     assert b"null pointer" in lib.vdn_last_error()
+    rows, cols = ctypes.c_int64(0), ctypes.c_int(0)
+    assert lib.vdn_mxfp8_gemm_plan(100, 128, 128, 0, ctypes.addressof(rows), ctypes.addressof(cols)) != 0
+    assert lib.vdn_mxfp8_gemm_plan(128, 128, 128, 4, ctypes.addressof(rows), ctypes.addressof(cols)) != 0
+    assert lib.vdn_mxfp8_gemm_plan(128, 128, 128, 0, None, ctypes.addressof(cols)) != 0
+    assert b"invalid argument" in lib.vdn_last_error()
 
 
 def test_short_conv_and_swiglu_entry_points_validate_before_launching():

@@ -1,6 +1,6 @@
 """The block-scaled GEMM's fused epilogues at the sizes the 108k block runs them.
 
-Padded M and N >= 1024 select the persistent kernel (bias, gated residual, written out of
+The sizes here take the persistent kernel (bias, gated residual, written out of
 place or over the residual) or, for an addend or rows not 16-byte aligned, the 256 x 256
 tile kernel. The block's [O | O_lin] GEMM (K = 10240) and FFN-down (K = 13824) run the
 gated residual in place over the hidden state; cross-O runs the residual without a gate.
@@ -20,6 +20,7 @@ import pytest
 import torch
 
 from oracle import mxfp8 as om
+from test_gemm_stream_gpu import assert_plan
 from vdn_amd import mxfp8 as vm
 
 pytestmark = pytest.mark.gpu
@@ -99,6 +100,8 @@ def test_persistent_residual_epilogue(device, k, in_place, with_gate):
     """The persistent kernel's residual epilogue (residual rows prefetched one 16-row group
     ahead), with and without the gate, out of place and over the residual itself. Rows of
     the buffer past M are never written."""
+    for kind in (0, 1):
+        assert_plan(M, N, k, kind, -(-M // 128) * 128, 0)
     op = operands(k)
     q, s, wq, ws = quantized(op, device)
     bias, gate = op["bias"].to(device), op["gate"].to(device) if with_gate else None

@@ -1,11 +1,12 @@
-"""The block-scaled GEMM's stream kernel (small and middle sizes) against the oracle.
+"""The block-scaled GEMM's planned kernels (the stream kernel of the small and middle sizes, the large
+kernel, and both in one call) against the oracle.
 
-Shapes reach its 128- and 256-column tiles, whole tiles only, K steps shared between workgroups
-(alone and beside whole tiles), the rows left below whole waves of the large kernel, padded
-columns past the last 256-column tile, single and odd K steps and the last partial rows. Each is
-checked on sampled rows against the exactly dequantized float64 GEMM, within the accumulation
-bound of tests/test_mxfp8_gpu.py::test_gemm_gated_residual_epilogue, for the bf16, gated-residual
-and producer epilogues; without a workspace the same problem runs unshared.
+Each shape names the kernels it is there for, and the test asserts that the plan takes them: the
+stream kernel's 128- and 256-column tiles, one and several tiles per workgroup, the rows left below
+whole waves of the large kernel, padded columns past the last 256-column tile, single and odd K steps
+and the last partial rows. Each is checked on sampled rows against the exactly dequantized float64
+GEMM, within the accumulation bound of tests/test_mxfp8_gpu.py::test_gemm_gated_residual_epilogue,
+for the bf16, gated-residual and producer epilogues.
 """
 import ctypes
 
@@ -19,17 +20,29 @@ from vdn_amd import mxfp8 as vm
 
 pytestmark = pytest.mark.gpu
 
+# (m, n, k, rows of the large kernel, columns of the stream kernel's tiles below them)
 SHAPES = [
-    (1, 128, 128),        # one tile, one K step
-    (77, 5120, 1152),     # few tiles: K shared, 9 steps in uneven parts
-    (130, 200, 384),      # an odd number of steps, n below its padding
-    (300, 1920, 640),     # padded N 1920: the last 256-column tile half past it
-    (512, 5120, 1024),    # 128-column tiles
-    (960, 5120, 768),     # 256-column tiles, one each
-    (1560, 5120, 1536),   # whole tiles and shared ones beside them
-    (2304, 7168, 384),    # more than one whole tile each
-    (3330, 5376, 1024),   # the large kernel, then the rows below its whole waves
+    (1, 128, 128, 0, 128),         # one tile, one K step
+    (77, 5120, 1152, 0, 128),      # few tiles, 9 K steps
+    (130, 200, 384, 0, 128),       # an odd number of steps, n below its padding
+    (300, 1920, 640, 0, 128),
+    (512, 5120, 1024, 0, 128),
+    (1560, 5120, 256, 0, 128),     # two whole rounds of the CUs and a third, partial one
+    (960, 5120, 768, 0, 256),      # one tile each
+    (960, 5200, 768, 0, 256),      # padded N 5248: the last 256-column tile half past it
+    (2304, 7168, 384, 0, 256),     # a whole round and a partial one
+    (2040, 8192, 1280, 2048, 0),   # the large kernel, the last rows past M
+    (2177, 8192, 2304, 2048, 128),  # the large kernel, then the rows below its whole wave
+    (4097, 5376, 3712, 3072, 256),
 ]
+
+
+def assert_plan(m, n, k, kind, large_rows, tile_cols):
+    """The kernels the size takes on this device, so that another choice cannot leave one untested."""
+    rows, cols = ctypes.c_int64(-1), ctypes.c_int(-1)
+    _lib.call("vdn_mxfp8_gemm_plan", -(-m // 128) * 128, -(-n // 128) * 128, -(-k // 128) * 128, kind,
+              ctypes.byref(rows), ctypes.byref(cols))
+    assert (rows.value, cols.value) == (large_rows, tile_cols)
 
 
 def operands(m, n, k):
@@ -56,8 +69,10 @@ def check(got, rows, ref, limit):
     assert (err <= limit).all(), float((err / limit).max())
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
-def test_stream_gemm_matches_oracle(device, m, n, k):
+@pytest.mark.parametrize("m,n,k,large_rows,tile_cols", SHAPES)
+def test_stream_gemm_matches_oracle(device, m, n, k, large_rows, tile_cols):
+    for kind in range(3):
+        assert_plan(m, n, k, kind, large_rows, tile_cols)
     x, w, bias, gate, res, rows, y, limit = operands(m, n, k)
     q, s = vm.quantize_activation(x.to(device))
     wq, ws = vm.quantize_activation(w.to(device))
@@ -79,20 +94,17 @@ def test_stream_gemm_matches_oracle(device, m, n, k):
         fq, fs = vm.mxfp8_gemm_act_quantize(q, s, wq, ws, n, rows=m, bias=b, act=act)
         rq, rs = fn(plain)[:2]
         assert torch.equal(fq, rq) and torch.equal(fs, rs), act
-    # the same problem without a workspace
-    again = torch.empty(m, n, dtype=torch.bfloat16, device=device)
-    if n % 8 == 0:
-        _lib.call("vdn_mxfp8_gemm", q.data_ptr(), s.data_ptr(), q.shape[0], wq.data_ptr(),
-                  ws.data_ptr(), wq.shape[0], q.shape[1], b.data_ptr(), None, 0, None, 0, None,
-                  again.data_ptr(), m, n, n, None, _lib.stream(again.device))
-        check(again, rows, y, limit)
 
 
-@pytest.mark.parametrize("m,f,k", [(77, 1280, 1152), (1560, 2560, 1536), (3330, 2816, 1024),
-                                   (260, 200, 128)])
-def test_stream_swiglu_matches_separate_passes(device, m, f, k):
+@pytest.mark.parametrize("m,f,k,large_rows", [(77, 1280, 1152, 0), (1560, 2560, 1536, 0),
+                                              (3330, 2816, 1024, 0), (260, 200, 128, 0),
+                                              (2040, 4096, 1280, 2048), (4097, 4000, 1024, 4224),
+                                              (4097, 4000, 2048, 4096)])
+def test_stream_swiglu_matches_separate_passes(device, m, f, k, large_rows):
     """The SwiGLU producer against the same interleaved GEMM, regrouped, and the stand-alone
-    producer: the same bytes, also where K is shared."""
+    producer: the same bytes, from the stream kernel, the large kernel (whole tiles, and ragged in
+    rows and columns) and both in one call."""
+    assert_plan(m, -(-f // 128) * 256, k, 3, large_rows, 0 if large_rows >= m else 256)
     g = torch.Generator().manual_seed(m + f)
     x = (torch.randn(m, k, generator=g) * 2).to(torch.bfloat16).to(device)
     w, b = vm.interleave_swiglu((torch.randn(2 * f, k, generator=g) * 0.05).to(torch.bfloat16),
@@ -108,8 +120,11 @@ def test_stream_swiglu_matches_separate_passes(device, m, f, k):
 
 
 def test_stream_gemm_flags_nonfinite(device):
-    """An inf in one row reaches the flag through whole and through shared tiles."""
-    for m, n, k in ((77, 1280, 1152), (512, 5120, 256)):
+    """An inf in the last row reaches the flag from the stream kernel, the large kernel and the
+    rows below it; as no row of the output it does not."""
+    for m, n, k, large_rows, tile_cols in ((77, 1280, 1152, 0, 128), (512, 5120, 256, 0, 128),
+                                           (2040, 8192, 1280, 2048, 0), (2177, 8192, 2304, 2048, 128)):
+        assert_plan(m, n, k, 0, large_rows, tile_cols)
         x = torch.ones(m, k, dtype=torch.bfloat16)
         x[m - 1] = 3e38
         q, s = vm.quantize_activation(x.to(device))

@@ -287,10 +287,11 @@ def random_mx(rows, kp, seed, lo=110, hi=140):
 
 
 @pytest.mark.parametrize("m,n,kp", [(128, 128, 128), (256, 384, 640), (1024, 1024, 512),
-                                    (1280, 1152, 384)])
+                                    (1280, 1152, 384), (1024, 5248, 256), (2048, 8192, 1280)])
 def test_gemm_scale_layout_stress(device, m, n, kp):
     """Independent per-(row, K-block) scales on both operands pin the MFMA lane layout and
-    the per-lane E8M0 scale selection."""
+    the per-lane E8M0 scale selection, in the stream kernel's 128- and 256-column tiles and, last,
+    the large kernel's."""
     ac, an = random_mx(m, kp, 1)
     wc, wn = random_mx(n, kp, 2)
     a_s, w_s = om.swizzle(an), om.swizzle(wn)
@@ -391,8 +392,9 @@ def test_gemm_gated_residual_epilogue(device, in_place):
                                        (1100, 1408, 512, None), (129, 200, 128, "gelu_tanh")])
 def test_gemm_producer_epilogue_matches_separate_passes(device, m, n, k, act):
     """The fused FFN producer (GEMM + bias -> act -> MXFP8 in the epilogue) writes the same
-    bytes as the GEMM's bf16 output fed to the stand-alone producer kernel. Shapes cover both
-    tile sizes, rows and columns past a 256 tile, and N not a multiple of 128."""
+    bytes as the GEMM's bf16 output fed to the stand-alone producer kernel. Shapes cover
+    rows and columns past a tile and N not a multiple of 128; each kernel by size:
+    tests/test_gemm_stream_gpu.py."""
     g = torch.Generator().manual_seed(m + n)
     x = (torch.randn(m, k, generator=g) * 2).to(torch.bfloat16).to(device)
     w = (torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16).to(device)
@@ -464,12 +466,13 @@ def test_gemm_reports_nonfinite_result(device):
 
 
 @pytest.mark.parametrize("m,f,k", [(1100, 640, 512), (2048, 704, 256), (300, 384, 256),
-                                   (1024, 520, 128)])
+                                   (1024, 520, 128), (2040, 4096, 1280)])
 def test_gemm_swiglu_producer_matches_separate_passes(device, m, f, k):
     """The fused SwiGLU producer (the up projection's a and g halves interleaved in 128-row
     blocks, met in the GEMM epilogue) writes the same bytes as the plain [a | g] GEMM fed to
-    the stand-alone SwiGLU producer (tp_ff_forward's two steps). Shapes cover the persistent
-    kernel, the small-problem path, a SwiGLU width not a multiple of 128 and rows past a tile."""
+    the stand-alone SwiGLU producer (tp_ff_forward's two steps). Shapes cover the stream
+    kernel, a SwiGLU width not a multiple of 128, rows past a tile and, last, the persistent
+    kernel."""
     g = torch.Generator().manual_seed(m + f)
     x = (torch.randn(m, k, generator=g) * 2).to(torch.bfloat16).to(device)
     w = (torch.randn(2 * f, k, generator=g) * 0.05).to(torch.bfloat16).to(device)

@@ -37,6 +37,7 @@ SIGNATURES = {
     "vdn_mxfp8_gemm_act_quantize_ws": [_ptr, _ptr, _i64, _ptr, _ptr, _i64, _i64, _ptr, _i32, _ptr,
                                        _ptr, _i64, _i64, _ptr, _ptr, _i64, _ptr],
     "vdn_mxfp8_gemm_workspace": [_i64, _i64, _i64, _i32, _ptr],
+    "vdn_mxfp8_gemm_plan": [_i64, _i64, _i64, _i32, _ptr, _ptr],
     "vdn_vda_prepare": [_ptr, _i64, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _ptr, _ptr],
     "vdn_vda_conv_prepare": [_ptr, _i32, _i64, _i64, _i32, _i32, _i32, _ptr, _ptr, _i32, _ptr,
                              _ptr],

@@ -86,5 +86,7 @@ int launch_persistent(const GemmArgs& g, hipStream_t stream);
 
 // mxfp8_gemm_stream.hip: the large kernel, the stream kernel or both, by size.
 int launch_gemm_planned(const GemmArgs& g, int mode, hipStream_t stream);
+// Its choice: rows of the large kernel, and tile columns of the stream kernel below them (0: none).
+void gemm_choice(int64_t mp, int64_t np, int64_t kp, int mode, int64_t* large_rows, int* tile_cols);
 
 }  // namespace vdn

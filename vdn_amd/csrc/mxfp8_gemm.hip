@@ -1188,3 +1188,15 @@ VDN_API int vdn_mxfp8_gemm_workspace(int64_t mp, int64_t np, int64_t kp, int kin
   *bytes = 0;
   return kOk;
 }
+
+VDN_API int vdn_mxfp8_gemm_plan(int64_t mp, int64_t np, int64_t kp, int kind, int64_t* large_rows,
+                                int* tile_cols) {
+  const char* name = "vdn_mxfp8_gemm_plan";
+  if (large_rows == nullptr || tile_cols == nullptr || mp <= 0 || np <= 0 || kp <= 0 || mp % 128 || np % 128 ||
+      kp % 128 || kind < 0 || kind > 3)
+    return set_error(kInvalidArgument, "%s: invalid argument", name);
+  if (gemm_too_large(mp, np, kp, kind == 3 || (mp >= 1024 && np >= 1024) ? 256 : 128))
+    return set_error(kUnsupported, "%s: problem too large for 32-bit tile offsets", name);
+  gemm_choice(mp, np, kp, kind, large_rows, tile_cols);
+  return kOk;
+}

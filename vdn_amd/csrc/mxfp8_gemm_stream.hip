@@ -675,6 +675,12 @@ GemmPlan plan_gemm(int64_t mp, int64_t np, int64_t kp, int mode) {
 
 }  // namespace
 
+void gemm_choice(int64_t mp, int64_t np, int64_t kp, int mode, int64_t* large_rows, int* tile_cols) {
+  const GemmPlan plan = plan_gemm(mp, np, kp, mode);
+  *large_rows = plan.large_rows;
+  *tile_cols = plan.large_rows < mp ? plan.stream.bn : 0;
+}
+
 int launch_gemm_planned(const GemmArgs& g, int mode, hipStream_t stream) {
   const GemmPlan plan = plan_gemm(g.mp, g.np, g.kp, mode);
   if (plan.large_rows > 0) {
