@@ -34,8 +34,8 @@ D = 128
 
 GEMMS = ("vdn_mxfp8_gemm", "vdn_mxfp8_gemm_act_quantize")
 VDA_ENTRIES = ("vdn_vda_statistics", "vdn_vda_factors", "vdn_vda_compose", "vdn_vda_scan",
-               "vdn_vda_log_prefix", "vdn_vda_gather", "vdn_vda_readout", "vdn_vda_readout_mxfp8",
-               "vdn_vda_readout_gated")
+               "vdn_vda_chunk_scan", "vdn_vda_log_prefix", "vdn_vda_gather", "vdn_vda_readout",
+               "vdn_vda_readout_mxfp8", "vdn_vda_readout_gated")
 ATTENTION = ("vdn_window_attention", "vdn_window_attention_mxfp8")
 # the VDA passes bounded by HBM (the factors and the scan are latency-bound: 128x128
 # eliminations and 30 serial frame steps)
@@ -95,6 +95,9 @@ def work(name, a, plans):
     if name == "vdn_vda_scan":
         chunks, heads = a[3], a[4]
         return 0.0, 4 * chunks * heads * D * D * 4
+    if name == "vdn_vda_chunk_scan":   # every frame's factors once, a bank entry per chunk, both ways
+        frames, heads, chunks = a[3], a[4], a[7]
+        return 0.0, 2 * (frames + chunks) * heads * D * D * 4
     if name == "vdn_vda_log_prefix":
         f, h = a[1], a[2]
         return 0.0, 2 * f * h * D * 4

@@ -99,3 +99,15 @@ def test_convert_linear_to_mxfp8_refuses_training_tied_and_device_weights():
     block.attn.orig.to_k.weight = block.attn.orig.to_q.weight
     with pytest.raises(ValueError, match="tied"):
         vm.convert_linear_to_mxfp8(model, enabled=True)
+
+
+def test_bench_times_every_entry_point_of_the_linear_branch():
+    """The branch's time is the sum over the entry points bench.py names: all of them, but those that
+    its workloads add by name or do not run. Each has its bytes counted."""
+    import bench
+    from vdn_amd import _lib
+    branch = {n for n in _lib.SIGNATURES if n.startswith("vdn_vda_")}
+    assert branch - set(bench.VDA_ENTRIES) == {"vdn_vda_prepare", "vdn_vda_conv_prepare", "vdn_vda_epilogue"}
+    for name in bench.VDA_ENTRIES:
+        flop, nbytes = bench.work(name, (1,) * len(_lib.SIGNATURES[name]), {})
+        assert nbytes > 0, name
