@@ -201,7 +201,7 @@ int vdn_vda_scan(const float* CT, const float* CI, const float* seed, int chunks
 
 /*
  * vdn_vda_compose followed by vdn_vda_scan (per_direction = 1) in one pass over the frames, without
- * the composed maps: bank [2, chunks, heads, 128, 128], chunk c covering frames starts[c] ..
+ * the composed maps (another fp32 order, no further from the float64 result): bank [2, chunks, heads, 128, 128], chunk c covering frames starts[c] ..
  * ends[c] - 1 (consecutive, from 0 to frames).
  */
 int vdn_vda_chunk_scan(const float* T, const float* J, const float* seed, int frames, int heads,

@@ -149,6 +149,31 @@ def test_chunk_scan_matches_fp64_and_composed_scan(device, frames, heads, cuts_o
                                atol=3e-6, rtol=3e-5)
 
 
+@pytest.mark.parametrize("frames,heads,size", [(6, 40, 3), (35, 56, 5), (64, 40, 8)])
+def test_chunk_scan_is_no_further_off_than_composing(device, frames, heads, size):
+    """The scan over the frames has as many serial fp32 products as frames, the composed one fewer:
+    its bank must not be further from the float64 scan for that."""
+    A, B, alpha = _stats(frames, heads, seed=frames)
+    t, inj = vv.paper_delta_factors(A.to(device), B.to(device), alpha.to(device))
+    seed = (torch.randn(heads, 128, 128, generator=torch.Generator().manual_seed(1)) * .3).to(device)
+    cuts = list(range(0, frames, size)) + [frames]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=device)
+    starts, ends, chunks = i32(cuts[:-1]), i32(cuts[1:]), len(cuts) - 1
+    one, ct, ci, two = (torch.empty((2, chunks, heads, 128, 128), device=device) for _ in range(4))
+    st = vv._stream(t)
+    vv._lib.call("vdn_vda_chunk_scan", t.data_ptr(), inj.data_ptr(), seed.data_ptr(), frames, heads,
+                 starts.data_ptr(), ends.data_ptr(), chunks, one.data_ptr(), st)
+    vv._lib.call("vdn_vda_compose", t.data_ptr(), inj.data_ptr(), heads, starts.data_ptr(),
+                 ends.data_ptr(), chunks, ct.data_ptr(), ci.data_ptr(), st)
+    vv._lib.call("vdn_vda_scan", ct.data_ptr(), ci.data_ptr(), seed.data_ptr(), chunks, heads, 1,
+                 two.data_ptr(), st)
+    n = 8                                            # heads compared
+    prefix, suffix = ov.scan(t.cpu()[:, :n], inj.cpu()[:, :n], seed.cpu()[:n])
+    ref = torch.stack((prefix[torch.tensor(cuts[1:]) - 1], suffix[cuts[:-1]]))
+    off = [float((b[:, :, :n].double().cpu() - ref).norm() / ref.norm()) for b in (one, two)]
+    assert off[0] <= off[1] < 2e-6, off
+
+
 def test_gather_zero_decay_irregular_bounds_no_bridge(device):
     frames, h = 9, 1
     t = (torch.eye(128).expand(frames, h, 128, 128).contiguous() * .9)

@@ -319,7 +319,10 @@ def _scan_frames(frames, heads, cuts):
     """Whether one scan over all the frames beats composing the chunks and scanning those. The
     scan's 16 x heads workgroups are all resident up to 64 heads and take about 6 us a frame; the
     composition holds two states per chunk, about 10 us a frame, in waves of 1024 workgroups, and
-    then scans the chunks (56 heads, 35 frames in 7 chunks: 333 + 67 us against 252)."""
+    then scans the chunks (56 heads, 35 frames in 7 chunks: 333 + 67 us against 250). It was faster
+    at every size measured that the rule gives it (5 to 120 frames, 24 to 128 heads), and at some
+    that it does not (35 frames in 7 chunks: 8 heads 74 us composed against 76, 16 heads 120
+    against 79)."""
     longest = max(b - a for a, b in zip(cuts[:-1], cuts[1:]))
     chunks = len(cuts) - 1
     waves = -(-16 * heads * chunks // 1024)
@@ -329,7 +332,9 @@ def _scan_frames(frames, heads, cuts):
 def paper_boundary_scan(transitions, injections, plan, text_state=None):
     """Chunk composition, then both directional scans: bank [2, C, H, D, D] fp32
     (paper_stack.py:202-236). bank[0, c] is the forward state after chunk c; bank[1, c] the
-    reverse state after chunk c (i.e. covering frames cuts[c]..F-1)."""
+    reverse state after chunk c (i.e. covering frames cuts[c]..F-1). The number of heads chooses
+    between two orders of the fp32 products (_scan_frames), so a head's last bits can differ
+    between calls with different numbers of heads."""
     _cuda(transitions, "transitions", torch.float32)
     _cuda(injections, "injections", torch.float32)
     if (transitions.ndim != 4 or transitions.shape != injections.shape
