@@ -137,6 +137,27 @@ def test_stream_gemm_flags_nonfinite(device):
         assert int(flag.item()) == 0
 
 
+@pytest.mark.parametrize("m,n,k,large_rows,tile_cols", [(77, 1280, 1152, 0, 128), (2040, 8192, 1280, 2048, 0),
+                                                        (2177, 8192, 2304, 2048, 128)])
+def test_padding_rows_of_the_operand_do_not_matter(device, m, n, k, large_rows, tile_cols):
+    """Codes and scales that are NaN in the operand's rows past M (empty_activation leaves them as the
+    memory was with zero_padding=False) reach neither the output nor the non-finite flag."""
+    assert_plan(m, n, k, 1, large_rows, tile_cols)
+    g = torch.Generator().manual_seed(m)
+    q, s = vm.quantize_activation(torch.randn(m, k, generator=g).to(torch.bfloat16).to(device))
+    wq, ws = vm.quantize_activation((torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16).to(device))
+    res = torch.randn(m, n, generator=g).to(torch.bfloat16).to(device)
+    dirty, scales = q.clone(), om.unswizzle(s.cpu().numpy(), *q.shape)
+    dirty[m:] = 0xff
+    scales[m:] = 0xff
+    ds = torch.from_numpy(om.swizzle(scales)).to(device)
+    flag = torch.zeros(1, dtype=torch.int32, device=device)
+    for r in (None, res):
+        ref = vm.mxfp8_gemm(q, s, wq, ws, n, rows=m, residual=r)
+        assert torch.equal(vm.mxfp8_gemm(dirty, ds, wq, ws, n, rows=m, residual=r, nonfinite=flag), ref)
+    assert int(flag.item()) == 0
+
+
 def wide(rows, k, g):
     """Normal values whose 32-column MXFP8 blocks lie up to 2^10 apart: their products' sums are far
     from exact in fp32, so another order of them shows."""

@@ -235,7 +235,7 @@ constexpr int kPrenormThreads = 64 * kPrenormRows;
 
 // Rows of exactly kCols = 512 kS (+ 256 with kHalf: a last slice in lanes 0 .. 31) columns, every
 // slice real, eight rows per workgroup, two
-// workgroups per CU (60 KB of LDS and at most 128 VGPRs each), so one's table staging and
+// workgroups per CU (up to 63 KB of LDS and at most 128 VGPRs each), so one's table staging and
 // load latency overlap the other's arithmetic; each wave issues its row's loads before the
 // table row is staged. The row index is wave-uniform, so every address is a scalar row base
 // plus a per-lane offset. The arithmetic is that of the general path in straight-line code.
