@@ -287,7 +287,9 @@ class HybridDiTBlock(nn.Module):
         return adaln_tables(temb, k["adaln_w"], k["adaln_b"], self.cfg.hidden)
 
     def _side_stream(self, device):
-        """One side stream per device, default priority."""
+        """The block's side stream, default priority, kept between calls (another device: a new one).
+        Each block has its own, and with it a pool of its own in the caching allocator, which its
+        first call fills."""
         if self._side is None or self._side.device != device:
             self._side = torch.cuda.Stream(device=device)
         return self._side
