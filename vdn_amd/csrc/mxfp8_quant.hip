@@ -723,6 +723,8 @@ VDN_API int vdn_mxfp8_prenorm_quantize(const void* x, int64_t rows, int64_t k, i
   const int64_t tab_align = tf ? 4 : 8;
   const bool wave_ok = vec && aligned16(weight) && aligned16(scale) && aligned16(shift) &&
                        scale_stride % tab_align == 0 && shift_stride % tab_align == 0;
+  // The widths measured on the straight-line rows: the blocks' hidden sizes (1536, 5120, 5376) and
+  // 1024, 2048, 4096. Other multiples of 256 would fit the template; they keep the general kernels.
   if (wave_ok) {
 #define VDN_PRENORM_FULL(S, HALF, CHAINS)                                                            \
     if (k == 512 * (S) + ((HALF) ? 256 : 0)) {                                                 \
